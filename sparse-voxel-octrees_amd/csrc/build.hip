@@ -1996,6 +1996,7 @@ int emit_tree(Arena &ar, const Geometry &g, uint64_t *leafKey, uint32_t *leafWor
     // parents (level D - 1): the depth octree_validate reports, D + 1. The
     // scatter checked every node's slot and child block against the array.
     out.depth = L ? D + 1 : 0;
+    out.levels = D;
     out.center[0] = float(g.dataW) * 0.5f / float(g.side);  // VoxelData::getCenter, VoxelData.cpp:297-303
     out.center[1] = float(g.dataH) * 0.5f / float(g.side);
     out.center[2] = float(g.dataD) * 0.5f / float(g.side);

@@ -70,22 +70,17 @@ __device__ __forceinline__ int stripe_y0(const FrameParams &p, int s) { return s
 __device__ __forceinline__ int stripe_y1(const FrameParams &p, int s) { return min((s + 1) * p.sh, p.height); }
 
 
-// One ray to completion; the leaf word (normal) is read only when Normal is set.
-// The frame kernels keep the whole restart stack in LDS (the fine pass measured
-// slower with the root's entry in registers). With Count, *passes counts the
-// loop passes.
-template <bool Lod, bool Normal, typename Idx, bool Count = false>
+// One ray to completion; the leaf word (normal) is read only when Normal is
+// set. With Count, *passes counts the loop passes.
+template <bool Lod, bool Normal, typename Addr, bool Count = false>
 __device__ __forceinline__ int trace(const uint32_t *__restrict__ tree, float ox, float oy, float oz, float dx, float dy,
-                                     float dz, float rayScale, const Stack<Idx> &stk, uint32_t &normal, float &t,
+                                     float dz, float rayScale, const PathStack<Addr> &path, uint32_t &normal, float &t,
                                      uint32_t *passes = nullptr) {
-    Ray<Idx> r;
+    Ray<Addr> r;
     ray_init(r, tree, ox, oy, oz, dx, dy, dz, rayScale);
-    Idx leaf = 0;
-    int code;
-    do {
-        code = ray_step<Lod, true, Idx, Normal, 0>(r, tree, stk, normal, t, leaf);  // camera rays are finite
-        if (Count) ++*passes;
-    } while (code == kRunning);
+    WalkEnd<Addr> end;
+    const int code = walk<Lod, Count, Addr>(r, tree, path, t, end, passes);  // camera rays are finite
+    if (Normal && code == kLeaf) normal = tree[end.leaf()];
     return code;
 }
 
@@ -99,9 +94,9 @@ __device__ __forceinline__ void frame_dir(const FrameParams &p, float dx, float 
     d[2] = vz * s;
 }
 
-template <typename Idx, int N>
+template <typename Addr, int N>
 __global__ void __launch_bounds__(64) coarse_kernel(const uint32_t *__restrict__ tree, const FrameSet<N> set,
-                                                    int64_t corners, unsigned blocksPerFrame, int slots) {
+                                                    int64_t corners, unsigned blocksPerFrame, int levels) {
     extern __shared__ __align__(16) unsigned char lds[];
     const unsigned f = N == 1 ? 0u : blockIdx.x / blocksPerFrame;
     const int64_t i = int64_t(blockIdx.x - f * blocksPerFrame) * blockDim.x + threadIdx.x;
@@ -119,19 +114,19 @@ __global__ void __launch_bounds__(64) coarse_kernel(const uint32_t *__restrict__
     for (int k = 0; k < ty; ++k) dy -= p.tileScale;
     float d[3];
     frame_dir(p, dx, dy, d);
-    Stack<Idx> stk(lds, 64, slots, int(threadIdx.x));
+    const PathStack<Addr> path(lds, 64, levels, int(threadIdx.x));
     uint32_t normal = 0;
     float t = 0.0f;
-    const int code = trace<true, false, Idx>(tree, p.px, p.py, p.pz, d[0], d[1], d[2], p.coarseScale, stk, normal, t);
+    const int code = trace<true, false, Addr>(tree, p.px, p.py, p.pz, d[0], d[1], d[2], p.coarseScale, path, normal, t);
     depth[i] = code != march::kMiss ? t : kTreeMiss;
 }
 
 //
 // Planned (one frame): the tiles in a tile plan's cost order (tile_order.hpp),
 // each filed by cost for the plan's next frame.
-template <typename Idx, int N, bool Planned = false>
+template <typename Addr, int N, bool Planned = false>
 __global__ void __launch_bounds__(64) fine_kernel(const uint32_t *__restrict__ tree, const FrameSet<N> set,
-                                                  unsigned tilesPerFrame, int slots, TileOrder o) {
+                                                  unsigned tilesPerFrame, int levels, TileOrder o) {
     extern __shared__ __align__(16) unsigned char lds[];
     const int64_t g = Planned ? int64_t(ordered_tile(o, int(blockIdx.x), int(threadIdx.x))) : int64_t(blockIdx.x);
     const unsigned f = N == 1 ? 0u : unsigned(g / tilesPerFrame);
@@ -164,12 +159,12 @@ __global__ void __launch_bounds__(64) fine_kernel(const uint32_t *__restrict__ t
             float d[3];
             frame_dir(p, dx, dy, d);
             const float m = dev::fmax_ref(minT - 0.03f, 0.0f);
-            Stack<Idx> stk(lds, 64, slots, lane);
+            const PathStack<Addr> path(lds, 64, levels, lane);
             uint32_t normal = 0;
             float t = 0.0f;
             float v = 0.0f;
-            const int code = trace<false, true, Idx, Planned>(tree, p.px + d[0] * m, p.py + d[1] * m, p.pz + d[2] * m,
-                                                              d[0], d[1], d[2], 0.0f, stk, normal, t, &passes);
+            const int code = trace<false, true, Addr, Planned>(tree, p.px + d[0] * m, p.py + d[1] * m, p.pz + d[2] * m,
+                                                              d[0], d[1], d[2], 0.0f, path, normal, t, &passes);
             if (code != march::kMiss) {
                 // shade, src/Main.cpp:81-90
                 float n[3], c;
@@ -287,29 +282,19 @@ int launch_frames(svo_octree &h, FrameSet<N> &set, int n, hipStream_t s, svo_til
     if (nulls) HIP_TRY(hipMallocAsync(&scratch, sizeof(float) * size_t(corners) * size_t(nulls), s));
     for (int f = 0, k = 0; f < n; ++f)
         if (!set.depth[f]) set.depth[f] = static_cast<float *>(scratch) + size_t(corners) * size_t(k++);
-    const int slots = lds_slots(h.depth, 0);  // the whole stack in LDS (Reg = 0)
-    const bool wide = h.words.size() >= (uint64_t(1) << 32);
-    const size_t lds = size_t(slots) * 64 * ((wide ? 8 : 4) + sizeof(float));
+    const PathLaunch L = path_launch(h);
     const dim3 cgrid(static_cast<unsigned>(cblocks * n)), fgrid(static_cast<unsigned>(tiles * n)), block(64);
-    const TileOrder none{};
-    if (!wide) {
-        hipLaunchKernelGGL((coarse_kernel<uint32_t, N>), cgrid, block, lds, s, h.dwords, set, corners, unsigned(cblocks),
-                           slots);
-        if (tiles && plan)
-            hipLaunchKernelGGL((fine_kernel<uint32_t, N, true>), fgrid, block, lds, s, h.dwords, set, unsigned(tiles),
-                               slots, next_order(*plan));
-        else if (tiles)
-            hipLaunchKernelGGL((fine_kernel<uint32_t, N>), fgrid, block, lds, s, h.dwords, set, unsigned(tiles), slots,
-                               none);
-    } else {
-        hipLaunchKernelGGL((coarse_kernel<uint64_t, N>), cgrid, block, lds, s, h.dwords, set, corners, unsigned(cblocks),
-                           slots);
-        if (tiles && plan)
-            hipLaunchKernelGGL((fine_kernel<uint64_t, N, true>), fgrid, block, lds, s, h.dwords, set, unsigned(tiles),
-                               slots, next_order(*plan));
-        else if (tiles)
-            hipLaunchKernelGGL((fine_kernel<uint64_t, N>), fgrid, block, lds, s, h.dwords, set, unsigned(tiles), slots,
-                               none);
+    const TileOrder o = plan ? next_order(*plan) : TileOrder{};
+    auto coarse = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, cgrid, block, L.lds, s, h.dwords, set, corners, unsigned(cblocks), L.levels);
+    };
+    auto fine = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, fgrid, block, L.lds, s, h.dwords, set, unsigned(tiles), L.levels, o);
+    };
+    L.wide ? coarse(coarse_kernel<uint64_t, N>) : coarse(coarse_kernel<uint32_t, N>);
+    if (tiles) {
+        if (!L.wide) plan ? fine(fine_kernel<uint32_t, N, true>) : fine(fine_kernel<uint32_t, N>);
+        else plan ? fine(fine_kernel<uint64_t, N, true>) : fine(fine_kernel<uint64_t, N>);
     }
     hipError_t e = hipGetLastError();
     if (scratch) (void)hipFreeAsync(scratch, s);

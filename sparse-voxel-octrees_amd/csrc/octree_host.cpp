@@ -44,7 +44,9 @@ struct Item {
 // pointers only point forward, so with that rule the check visits each word
 // at most once. With `frontier`, nodes at level `split` are handed out
 // instead of descended into.
-int validate_from(const uint32_t *w, uint64_t n, Item root, int split, std::vector<Item> *frontier, uint64_t *seen) {
+// *levels receives the levels of descriptors visited, childless ones included.
+int validate_from(const uint32_t *w, uint64_t n, Item root, int split, std::vector<Item> *frontier, uint64_t *seen,
+                  int &levels) {
     std::vector<Item> stack;
     stack.push_back(root);
     int depth = 0;
@@ -56,6 +58,7 @@ int validate_from(const uint32_t *w, uint64_t n, Item root, int split, std::vect
             frontier->push_back(it);
             continue;
         }
+        levels = std::max(levels, it.level + 1);
         uint32_t d = w[it.idx];
         uint32_t valid = (d >> 8) & 0xFFu, nonleaf = d & 0xFFu;
         uint64_t per = 1 + ((d >> 16) & 1u);
@@ -98,7 +101,7 @@ int validate_from(const uint32_t *w, uint64_t n, Item root, int split, std::vect
 // (levels of descriptors + 1), -1 for a malformed tree or -2 when the check's
 // bitmap (one bit per word) cannot be allocated. Subtrees below level 3 are
 // checked on all host threads.
-int octree_validate(const uint32_t *w, uint64_t n) {
+int octree_validate(const uint32_t *w, uint64_t n, int *levelsOut) {
     if (n == 0) return -1;
     // the root's child offset, far form included: the traversal reads it like
     // any other descriptor's (src/VoxelOctree.cpp:276-280)
@@ -115,22 +118,28 @@ int octree_validate(const uint32_t *w, uint64_t n) {
     seen[0] = 1;  // the root
     std::vector<Item> frontier;
     const int split = 3;
-    int depth = validate_from(w, n, {0, rootOff, 0}, split, &frontier, seen);
+    int levels = 1;
+    int depth = validate_from(w, n, {0, rootOff, 0}, split, &frontier, seen, levels);
     if (depth < 0) return -1;
     depth = std::max(depth, 1);
+    if (levelsOut) *levelsOut = levels;
     if (frontier.empty()) return depth;
     std::atomic<size_t> next{0};
-    std::atomic<int> worst{depth};
+    std::atomic<int> worst{depth}, most{levels};
     std::atomic<bool> bad{false};
     auto worker = [&]() {
         for (size_t i; !bad.load() && (i = next.fetch_add(1)) < frontier.size();) {
-            int d = validate_from(w, n, frontier[i], split, nullptr, seen);
+            int lv = 1;
+            int d = validate_from(w, n, frontier[i], split, nullptr, seen, lv);
             if (d < 0) {
                 bad.store(true);
                 return;
             }
             int cur = worst.load();
             while (d > cur && !worst.compare_exchange_weak(cur, d)) {
+            }
+            cur = most.load();
+            while (lv > cur && !most.compare_exchange_weak(cur, lv)) {
             }
         }
     };
@@ -142,6 +151,7 @@ int octree_validate(const uint32_t *w, uint64_t n) {
     }
     worker();
     for (std::thread &t : pool) t.join();
+    if (levelsOut) *levelsOut = most.load();
     return bad.load() ? -1 : worst.load();
 }
 

@@ -12,6 +12,7 @@
 //  - word indices are 32-bit when the tree has < 2^32 words, else 64-bit.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <mutex>
@@ -33,21 +34,20 @@ namespace {
 
 using namespace march;
 
-// Runs one ray to completion. Returns 0 miss, 1 leaf hit, 2 LOD hit. With
-// Normal set, a leaf hit also gives the leaf's word index and word.
-// With Count, *passes counts the loop passes.
-template <bool Lod, bool Finite, typename Idx, bool Normal = true, int Reg = 1, bool Count = false>
+// Walks one finite ray to its end: 0 miss, 1 leaf hit (with its word index and
+// word when Normal is set), 2 LOD hit. With Count, *passes counts the passes.
+template <bool Lod, typename Addr, bool Normal = true, bool Count = false>
 __device__ __forceinline__ int march_ray(const uint32_t *__restrict__ tree, float ox, float oy, float oz, float dx,
-                                         float dy, float dz, float rayScale, const Stack<Idx> &stk, uint32_t &normal,
-                                         float &tOut, Idx &leaf, uint32_t *passes = nullptr) {
-    Ray<Idx> r;
+                                         float dy, float dz, float rayScale, const PathStack<Addr> &path,
+                                         uint32_t &normal, float &tOut, Addr &leaf, uint32_t *passes = nullptr) {
+    Ray<Addr> r;
     ray_init(r, tree, ox, oy, oz, dx, dy, dz, rayScale);
-    if (!Finite && !ray_defined(r)) return kMiss;  // the reference never ends such a ray
-    int code;
-    do {
-        code = ray_step<Lod, Finite, Idx, Normal, Reg>(r, tree, stk, normal, tOut, leaf);
-        if (Count) ++*passes;
-    } while (code == kRunning);
+    WalkEnd<Addr> end;
+    const int code = walk<Lod, Count, Addr>(r, tree, path, tOut, end, passes);
+    if (Normal && code == kLeaf) {
+        leaf = end.leaf();
+        normal = tree[leaf];
+    }
     return code;
 }
 
@@ -60,23 +60,35 @@ __device__ __forceinline__ void store_result(int code, uint32_t normal, float t,
     if (lf) lf[i] = code == 1 ? uint64_t(leaf) : SVO_LEAF_NONE;
 }
 
-template <typename Idx>
-__global__ void __launch_bounds__(256) rays_kernel(const uint32_t *__restrict__ tree, int64_t n,
-                                                   const float *__restrict__ o, const float *__restrict__ d,
-                                                   const float *__restrict__ rs, float rs0, int slots,
-                                                   uint8_t *hit, uint32_t *nrm, float *tt, uint64_t *lf) {
+// Arbitrary caller rays, one wave per 64: finite rays take the walk, the
+// others the reference's loop step by step (exact std::min and NaN semantics).
+template <bool Lod, typename Addr>
+__global__ void __launch_bounds__(64) rays_kernel(const uint32_t *__restrict__ tree, int64_t n,
+                                                  const float *__restrict__ o, const float *__restrict__ d,
+                                                  const float *__restrict__ rs, float rs0, int levels, int slots,
+                                                  uint8_t *hit, uint32_t *nrm, float *tt, uint64_t *lf) {
     extern __shared__ __align__(16) unsigned char lds[];
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    const int64_t i = int64_t(blockIdx.x) * 64 + threadIdx.x;
     if (i >= n) return;
-    Stack<Idx> stk(lds, int(blockDim.x), slots, int(threadIdx.x));
     uint32_t normal = 0;
     float t = 0.0f;
-    Idx leaf = 0;
-    const float scale = rs ? rs[i] : rs0;
-    // arbitrary caller rays: LOD test kept, exact std::min semantics
-    int code = march_ray<true, false, Idx>(tree, o[3 * i], o[3 * i + 1], o[3 * i + 2], d[3 * i], d[3 * i + 1],
-                                           d[3 * i + 2], scale, stk, normal, t, leaf);
-    store_result<Idx>(code, normal, t, leaf, i, hit, nrm, tt, lf);
+    Addr leaf = 0;
+    const float scale = Lod && rs ? rs[i] : rs0;
+    const float ox = o[3 * i], oy = o[3 * i + 1], oz = o[3 * i + 2], dx = d[3 * i], dy = d[3 * i + 1], dz = d[3 * i + 2];
+    int code = kMiss;
+    if (ray_finite(ox, oy, oz, dx, dy, dz)) {
+        const PathStack<Addr> path(lds, 64, levels, int(threadIdx.x));
+        code = march_ray<Lod, Addr>(tree, ox, oy, oz, dx, dy, dz, scale, path, normal, t, leaf);
+    } else {
+        const Stack<Addr> stk(lds, 64, slots, int(threadIdx.x));
+        Ray<Addr> r;
+        ray_init(r, tree, ox, oy, oz, dx, dy, dz, scale);
+        if (ray_defined(r))  // the reference never ends the other rays
+            do {
+                code = ray_step<true, false, Addr, true, 3>(r, tree, stk, normal, t, leaf);
+            } while (code == kRunning);
+    }
+    store_result<Addr>(code, normal, t, leaf, i, hit, nrm, tt, lf);
 }
 
 struct PrimaryParams {
@@ -101,9 +113,9 @@ __device__ __forceinline__ void primary_dir(const PrimaryParams &p, int x, int y
 }
 
 // 8x8 pixel tile per wave64; lanes raster the tile row by row.
-template <typename Idx, int Reg>
+template <typename Addr>
 __global__ void __launch_bounds__(64) primary_kernel(const uint32_t *__restrict__ tree, PrimaryParams p,
-                                                     int slots, uint8_t *hit, uint32_t *nrm, float *tt,
+                                                     int levels, uint8_t *hit, uint32_t *nrm, float *tt,
                                                      uint64_t *lf) {
     extern __shared__ __align__(16) unsigned char lds[];
     const int tile = int(blockIdx.x);
@@ -113,20 +125,19 @@ __global__ void __launch_bounds__(64) primary_kernel(const uint32_t *__restrict_
     if (x >= p.width || y >= p.height) return;
     float d[3];
     primary_dir(p, x, y, d);
-    Stack<Idx> stk(lds, 64, slots, lane);
+    const PathStack<Addr> path(lds, 64, levels, lane);
     uint32_t normal = 0;
     float t = 0.0f;
-    Idx leaf = 0;
-    int code = march_ray<false, true, Idx, true, Reg>(tree, p.px, p.py, p.pz, d[0], d[1], d[2], 0.0f, stk, normal, t,
-                                                      leaf);
-    store_result<Idx>(code, normal, t, leaf, int64_t(y) * p.width + x, hit, nrm, tt, lf);
+    Addr leaf = 0;
+    const int code = march_ray<false, Addr>(tree, p.px, p.py, p.pz, d[0], d[1], d[2], 0.0f, path, normal, t, leaf);
+    store_result<Addr>(code, normal, t, leaf, int64_t(y) * p.width + x, hit, nrm, tt, lf);
 }
 
 // Cost-ordered form of primary_kernel (tile_order.hpp): workgroup b traces the
 // tile the plan's order gives and files it by cost for the next launch.
-template <typename Idx, int Reg>
+template <typename Addr>
 __global__ void __launch_bounds__(64) primary_ordered_kernel(const uint32_t *__restrict__ tree, PrimaryParams p,
-                                                             int slots, TileOrder o, uint8_t *hit, uint32_t *nrm,
+                                                             int levels, TileOrder o, uint8_t *hit, uint32_t *nrm,
                                                              float *tt, uint64_t *lf) {
     extern __shared__ __align__(16) unsigned char lds[];
     const int lane = threadIdx.x;
@@ -137,18 +148,13 @@ __global__ void __launch_bounds__(64) primary_ordered_kernel(const uint32_t *__r
     if (x < p.width && y < p.height) {
         float d[3];
         primary_dir(p, x, y, d);
-        Stack<Idx> stk(lds, 64, slots, lane);
-        Ray<Idx> r;
-        ray_init(r, tree, p.px, p.py, p.pz, d[0], d[1], d[2], 0.0f);
+        const PathStack<Addr> path(lds, 64, levels, lane);
         uint32_t normal = 0;
         float t = 0.0f;
-        Idx leaf = 0;
-        int code;
-        do {
-            code = ray_step<false, true, Idx, true, Reg>(r, tree, stk, normal, t, leaf);
-            passes++;
-        } while (code == kRunning);
-        store_result<Idx>(code, normal, t, leaf, int64_t(y) * p.width + x, hit, nrm, tt, lf);
+        Addr leaf = 0;
+        const int code = march_ray<false, Addr, true, true>(tree, p.px, p.py, p.pz, d[0], d[1], d[2], 0.0f, path,
+                                                            normal, t, leaf, &passes);
+        store_result<Addr>(code, normal, t, leaf, int64_t(y) * p.width + x, hit, nrm, tt, lf);
     }
     file_tile(o, int(blockIdx.x), tile, passes, lane);
 }
@@ -166,9 +172,9 @@ __global__ void __launch_bounds__(64) primary_ordered_kernel(const uint32_t *__r
 //
 // Planned: the tiles in a tile plan's cost order (tile_order.hpp), each filed
 // by its primary plus shadow passes for the plan's next launch.
-template <typename Idx, int Reg, bool Planned = false>
+template <typename Addr, bool Planned = false>
 __global__ void __launch_bounds__(64) primary_shadow_kernel(const uint32_t *__restrict__ tree, PrimaryParams p,
-                                                            float lx, float ly, float lz, float eps, int slots,
+                                                            float lx, float ly, float lz, float eps, int levels,
                                                             uint8_t *hit, uint32_t *nrm, float *tt, uint64_t *lf,
                                                             uint8_t *__restrict__ shadow, TileOrder o) {
     extern __shared__ __align__(16) unsigned char lds[];
@@ -180,23 +186,23 @@ __global__ void __launch_bounds__(64) primary_shadow_kernel(const uint32_t *__re
     if (x < p.width && y < p.height) {
         float d[3];
         primary_dir(p, x, y, d);
-        Stack<Idx> stk(lds, 64, slots, lane);
+        const PathStack<Addr> path(lds, 64, levels, lane);
         uint32_t normal = 0;
         float t = 0.0f;
-        Idx leaf = 0;
-        const int code = march_ray<false, true, Idx, true, Reg, Planned>(tree, p.px, p.py, p.pz, d[0], d[1], d[2], 0.0f,
-                                                                         stk, normal, t, leaf, &passes);
+        Addr leaf = 0;
+        const int code = march_ray<false, Addr, true, Planned>(tree, p.px, p.py, p.pz, d[0], d[1], d[2], 0.0f, path,
+                                                               normal, t, leaf, &passes);
         const int64_t i = int64_t(y) * p.width + x;
-        store_result<Idx>(code, normal, t, leaf, i, hit, nrm, tt, lf);
+        store_result<Addr>(code, normal, t, leaf, i, hit, nrm, tt, lf);
         uint8_t sh = 0;
         if (code == 1) {
             const float back = t - eps;
             uint32_t n2 = 0;
             float t2 = 0.0f;
-            Idx leaf2 = 0;
-            const int c2 = march_ray<false, true, Idx, false, Reg, Planned>(tree, p.px + d[0] * back, p.py + d[1] * back,
-                                                                            p.pz + d[2] * back, lx, ly, lz, 0.0f, stk,
-                                                                            n2, t2, leaf2, &passes);
+            Addr leaf2 = 0;
+            const int c2 = march_ray<false, Addr, false, Planned>(tree, p.px + d[0] * back, p.py + d[1] * back,
+                                                                  p.pz + d[2] * back, lx, ly, lz, 0.0f, path, n2, t2,
+                                                                  leaf2, &passes);
             sh = (c2 == 1 || c2 == 2) ? 1 : 0;
         }
         shadow[i] = sh;
@@ -204,14 +210,12 @@ __global__ void __launch_bounds__(64) primary_shadow_kernel(const uint32_t *__re
     if (Planned) file_tile(o, int(blockIdx.x), tile, passes, lane);
 }
 
-int stack_slots(const svo_octree &h, int reg) { return lds_slots(h.depth, reg); }
-
 template <typename Idx>
 int walk_one(const svo_octree &h, const float o[3], const float d[3], float rs, uint32_t &normal, float &t,
              uint64_t &leaf) {
     const uint32_t *tree = h.words.data();
     uint64_t buf[48];  // the restart stack: at most 21 entries of (index, maxT)
-    const Stack<Idx> stk(buf, 1, stack_slots(h, 1), 0);
+    const Stack<Idx> stk(buf, 1, lds_slots(h.depth, 1), 0);
     Ray<Idx> r;
     ray_init(r, tree, o[0], o[1], o[2], d[0], d[1], d[2], rs);
     if (!ray_defined(r)) return kMiss;  // the reference never ends such a ray
@@ -233,6 +237,14 @@ int raymarch_one(const svo_octree &h, const float o[3], const float d[3], float 
                  uint64_t &leaf) {
     if (h.words.size() < (uint64_t(1) << 32)) return walk_one<uint32_t>(h, o, d, rs, normal, t, leaf);
     return walk_one<uint64_t>(h, o, d, rs, normal, t, leaf);
+}
+
+PathLaunch path_launch(const svo_octree &h) {
+    PathLaunch L;
+    L.levels = h.levels;
+    L.wide = h.words.size() >= (uint64_t(1) << 30);
+    L.lds = L.wide ? path_bytes<uint64_t>(L.levels) : path_bytes<uint32_t>(L.levels);
+    return L;
 }
 
 int device_count() {
@@ -280,19 +292,19 @@ int raymarch_device(svo_octree &h, int64_t n, const float *o, const float *d, co
     if (!o || !d) return fail(SVO_ERR_INVALID, "null ray arrays");
     int r = ensure_device(h);
     if (r) return r;
-    const int threads = 256;
-    const int slots = stack_slots(h, 1);
-    const bool wide = h.words.size() >= (uint64_t(1) << 32);
-    const size_t lds = size_t(slots) * threads * ((wide ? 8 : 4) + sizeof(float));
-    const int64_t blocks = (n + threads - 1) / threads;
+    const int64_t blocks = (n + 63) / 64;
     if (blocks > 0x7FFFFFFF) return fail(SVO_ERR_LIMIT, "too many rays for one launch");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (!wide)
-        hipLaunchKernelGGL(rays_kernel<uint32_t>, dim3(unsigned(blocks)), dim3(threads), lds, s, h.dwords, n, o, d,
-                           rs, rs0, slots, hit, normal, t, leaf);
-    else
-        hipLaunchKernelGGL(rays_kernel<uint64_t>, dim3(unsigned(blocks)), dim3(threads), lds, s, h.dwords, n, o, d,
-                           rs, rs0, slots, hit, normal, t, leaf);
+    const PathLaunch L = path_launch(h);
+    const int slots = lds_slots(h.depth, 3);
+    const size_t lds = std::max(L.lds, size_t(slots) * 64 * ((L.wide ? 8 : 4) + sizeof(float)));
+    const bool lod = rs || rs0 != 0.0f;
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(unsigned(blocks)), dim3(64), lds, s, h.dwords, n, o, d, rs, rs0, L.levels, slots,
+                           hit, normal, t, leaf);
+    };
+    if (!L.wide) lod ? launch(rays_kernel<true, uint32_t>) : launch(rays_kernel<false, uint32_t>);
+    else lod ? launch(rays_kernel<true, uint64_t>) : launch(rays_kernel<false, uint64_t>);
     HIP_TRY(hipGetLastError());
     return SVO_OK;
 }
@@ -322,34 +334,14 @@ PrimaryParams primary_params(const svo_camera &cam, int width, int height) {
 
 namespace {
 
-// Launch shape shared by the primary and shadow passes of one octree.
-struct TileLaunch {
-    int reg, slots;
-    bool wide;
-    size_t lds;
-};
-
-TileLaunch tile_launch(const svo_octree &h) {
-    TileLaunch L;
-    L.reg = reg_entries(h.depth);
-    L.slots = stack_slots(h, L.reg);
-    L.wide = h.words.size() >= (uint64_t(1) << 32);
-    L.lds = size_t(L.slots) * 64 * ((L.wide ? 8 : 4) + sizeof(float));
-    return L;
-}
-
 // The primary pass over every tile of the image, one wave per 8x8 tile.
-void launch_primary(const svo_octree &h, const TileLaunch &L, const PrimaryParams &p, int tiles, uint8_t *hit,
+void launch_primary(const svo_octree &h, const PathLaunch &L, const PrimaryParams &p, int tiles, uint8_t *hit,
                     uint32_t *normal, float *t, uint64_t *leaf, hipStream_t s) {
     const dim3 grid(static_cast<unsigned>(tiles)), block(64);
-    if (!L.wide && L.reg == 1)
-        hipLaunchKernelGGL((primary_kernel<uint32_t, 1>), grid, block, L.lds, s, h.dwords, p, L.slots, hit, normal, t, leaf);
-    else if (!L.wide)
-        hipLaunchKernelGGL((primary_kernel<uint32_t, 3>), grid, block, L.lds, s, h.dwords, p, L.slots, hit, normal, t, leaf);
-    else if (L.reg == 1)
-        hipLaunchKernelGGL((primary_kernel<uint64_t, 1>), grid, block, L.lds, s, h.dwords, p, L.slots, hit, normal, t, leaf);
+    if (!L.wide)
+        hipLaunchKernelGGL(primary_kernel<uint32_t>, grid, block, L.lds, s, h.dwords, p, L.levels, hit, normal, t, leaf);
     else
-        hipLaunchKernelGGL((primary_kernel<uint64_t, 3>), grid, block, L.lds, s, h.dwords, p, L.slots, hit, normal, t, leaf);
+        hipLaunchKernelGGL(primary_kernel<uint64_t>, grid, block, L.lds, s, h.dwords, p, L.levels, hit, normal, t, leaf);
 }
 
 }  // namespace
@@ -396,18 +388,6 @@ void tile_plan_free(svo_tile_plan *p) {
     delete p;
 }
 
-namespace {
-
-template <typename Idx, int Reg>
-void launch_ordered(const svo_octree &h, const TileLaunch &L, const PrimaryParams &p, const svo_tile_plan &plan,
-                    uint8_t *hit, uint32_t *normal, float *t, uint64_t *leaf, hipStream_t s) {
-    const TileOrder o = next_order(plan);
-    hipLaunchKernelGGL((primary_ordered_kernel<Idx, Reg>), dim3(unsigned(plan.tiles)), dim3(64), L.lds, s, h.dwords, p,
-                       L.slots, o, hit, normal, t, leaf);
-}
-
-}  // namespace
-
 int render_primary_planned_device(svo_octree &h, svo_tile_plan *plan, const svo_camera &cam, int width, int height,
                                   uint8_t *hit, uint32_t *normal, float *t, uint64_t *leaf, void *stream) {
     if (!plan) return fail(SVO_ERR_INVALID, "null tile plan");
@@ -420,12 +400,16 @@ int render_primary_planned_device(svo_octree &h, svo_tile_plan *plan, const svo_
     int r = ensure_device(h);
     if (r) return r;
     const PrimaryParams p = primary_params(cam, width, height);
-    const TileLaunch L = tile_launch(h);
+    const PathLaunch L = path_launch(h);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (!L.wide && L.reg == 1) launch_ordered<uint32_t, 1>(h, L, p, *plan, hit, normal, t, leaf, s);
-    else if (!L.wide) launch_ordered<uint32_t, 3>(h, L, p, *plan, hit, normal, t, leaf, s);
-    else if (L.reg == 1) launch_ordered<uint64_t, 1>(h, L, p, *plan, hit, normal, t, leaf, s);
-    else launch_ordered<uint64_t, 3>(h, L, p, *plan, hit, normal, t, leaf, s);
+    const TileOrder order = next_order(*plan);
+    const dim3 grid(unsigned(plan->tiles)), block(64);
+    if (!L.wide)
+        hipLaunchKernelGGL(primary_ordered_kernel<uint32_t>, grid, block, L.lds, s, h.dwords, p, L.levels, order, hit,
+                           normal, t, leaf);
+    else
+        hipLaunchKernelGGL(primary_ordered_kernel<uint64_t>, grid, block, L.lds, s, h.dwords, p, L.levels, order, hit,
+                           normal, t, leaf);
     HIP_TRY(hipGetLastError());
     plan->renders++;
     return SVO_OK;
@@ -440,7 +424,7 @@ int render_primary_device(svo_octree &h, const svo_camera &cam, int width, int h
     if (r) return r;
     const PrimaryParams p = primary_params(cam, width, height);
     const int tiles = p.tilesX * ((height + 7) / 8);
-    launch_primary(h, tile_launch(h), p, tiles, hit, normal, t, leaf, static_cast<hipStream_t>(stream));
+    launch_primary(h, path_launch(h), p, tiles, hit, normal, t, leaf, static_cast<hipStream_t>(stream));
     HIP_TRY(hipGetLastError());
     return SVO_OK;
 }
@@ -471,36 +455,15 @@ int render_shadow_device(svo_octree &h, const svo_camera &cam, int width, int he
     if (r) return r;
     const PrimaryParams p = primary_params(cam, width, height);
     const int tiles = p.tilesX * ((height + 7) / 8);
-    const TileLaunch L = tile_launch(h);
+    const PathLaunch L = path_launch(h);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const dim3 grid(static_cast<unsigned>(tiles)), block(64);
     const TileOrder o = plan ? next_order(*plan) : TileOrder{};
-    if (plan) {
-        if (!L.wide && L.reg == 1)
-            hipLaunchKernelGGL((primary_shadow_kernel<uint32_t, 1, true>), grid, block, L.lds, s, h.dwords, p, light[0],
-                               light[1], light[2], eps, L.slots, hit, normal, t, leaf, shadow, o);
-        else if (!L.wide)
-            hipLaunchKernelGGL((primary_shadow_kernel<uint32_t, 3, true>), grid, block, L.lds, s, h.dwords, p, light[0],
-                               light[1], light[2], eps, L.slots, hit, normal, t, leaf, shadow, o);
-        else if (L.reg == 1)
-            hipLaunchKernelGGL((primary_shadow_kernel<uint64_t, 1, true>), grid, block, L.lds, s, h.dwords, p, light[0],
-                               light[1], light[2], eps, L.slots, hit, normal, t, leaf, shadow, o);
-        else
-            hipLaunchKernelGGL((primary_shadow_kernel<uint64_t, 3, true>), grid, block, L.lds, s, h.dwords, p, light[0],
-                               light[1], light[2], eps, L.slots, hit, normal, t, leaf, shadow, o);
-    } else if (!L.wide && L.reg == 1) {
-        hipLaunchKernelGGL((primary_shadow_kernel<uint32_t, 1>), grid, block, L.lds, s, h.dwords, p, light[0], light[1],
-                           light[2], eps, L.slots, hit, normal, t, leaf, shadow, o);
-    } else if (!L.wide) {
-        hipLaunchKernelGGL((primary_shadow_kernel<uint32_t, 3>), grid, block, L.lds, s, h.dwords, p, light[0], light[1],
-                           light[2], eps, L.slots, hit, normal, t, leaf, shadow, o);
-    } else if (L.reg == 1) {
-        hipLaunchKernelGGL((primary_shadow_kernel<uint64_t, 1>), grid, block, L.lds, s, h.dwords, p, light[0], light[1],
-                           light[2], eps, L.slots, hit, normal, t, leaf, shadow, o);
-    } else {
-        hipLaunchKernelGGL((primary_shadow_kernel<uint64_t, 3>), grid, block, L.lds, s, h.dwords, p, light[0], light[1],
-                           light[2], eps, L.slots, hit, normal, t, leaf, shadow, o);
-    }
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(unsigned(tiles)), dim3(64), L.lds, s, h.dwords, p, light[0], light[1], light[2], eps,
+                           L.levels, hit, normal, t, leaf, shadow, o);
+    };
+    if (!L.wide) plan ? launch(primary_shadow_kernel<uint32_t, true>) : launch(primary_shadow_kernel<uint32_t>);
+    else plan ? launch(primary_shadow_kernel<uint64_t, true>) : launch(primary_shadow_kernel<uint64_t>);
     HIP_TRY(hipGetLastError());
     if (plan) plan->renders++;
     return SVO_OK;

@@ -187,10 +187,10 @@ __global__ void __launch_bounds__(256) batch_kernel(const ViewDesc *__restrict__
 //
 // Planned: the batch's tiles in a tile plan's cost order (tile_order.hpp),
 // each filed by cost for the plan's next launch; one launch (first = 0).
-template <bool Lod, typename Idx, int Reg, bool Planned = false>
+template <bool Lod, typename Addr, bool Planned = false>
 __global__ void __launch_bounds__(64) tiles_kernel(const ViewDesc *__restrict__ views,
                                                    const uint64_t *__restrict__ tileBase, int nviews, uint64_t first,
-                                                   int slots, int twLog, TileOrder o) {
+                                                   int levels, int twLog, TileOrder o) {
     extern __shared__ __align__(16) unsigned char lds[];
     const int lane = threadIdx.x;
     const uint64_t tile = Planned ? uint64_t(ordered_tile(o, int(blockIdx.x), lane)) : first + blockIdx.x;
@@ -207,18 +207,19 @@ __global__ void __launch_bounds__(64) tiles_kernel(const ViewDesc *__restrict__ 
     if (inside) {
         float dx, dy, dz;
         view_ray_dir(vd, x, y, dx, dy, dz);
-        Stack<Idx> stk(lds, 64, slots, lane);
-        Ray<Idx> r;
+        const PathStack<Addr> path(lds, 64, levels, lane);
+        Ray<Addr> r;
         ray_init(r, vd.tree, vd.px, vd.py, vd.pz, dx, dy, dz, vd.rayScale);
+        WalkEnd<Addr> end;
         uint32_t normal = 0;
         float t = 0.0f;
-        Idx leaf = 0;
-        int code;
-        do {
-            code = ray_step<Lod, true, Idx, true, Reg>(r, vd.tree, stk, normal, t, leaf);
-            if (Planned) passes++;
-        } while (code == kRunning);
-        view_store<Idx>(vd, int64_t(y) * vd.width + x, code, normal, t, leaf);
+        Addr leaf = 0;
+        const int code = walk<Lod, Planned, Addr>(r, vd.tree, path, t, end, &passes);
+        if (code == kLeaf) {
+            leaf = end.leaf();
+            normal = vd.tree[leaf];
+        }
+        view_store<Addr>(vd, int64_t(y) * vd.width + x, code, normal, t, leaf);
     }
     if (Planned) file_tile(o, int(blockIdx.x), int(tile), passes, lane);
 }
@@ -338,7 +339,7 @@ int tile_width_log(int w) {
 // view of an octree not resident on the current device is refused).
 int plan_views(const svo_view *views, int nviews, const svo_batch_opts *opts, int cus, ViewDesc *hv, uint64_t *htb,
                LaunchPlan &plan, bool upload) {
-    int maxDepth = 1;
+    int maxDepth = 1, maxLevels = 1;
     bool wide = false, lod = false;
     uint64_t tiles = 0;
     const bool persistentForm = opts && opts->form == SVO_BATCH_PERSISTENT;
@@ -362,7 +363,9 @@ int plan_views(const svo_view *views, int nviews, const svo_batch_opts *opts, in
         if (r) return r;
         lod = lod || v.ray_scale != 0.0f;
         maxDepth = std::max(maxDepth, v.tree->depth);
-        wide = wide || v.tree->words.size() >= (uint64_t(1) << 32);
+        const PathLaunch pl = path_launch(*v.tree);
+        maxLevels = std::max(maxLevels, pl.levels);
+        wide = wide || pl.wide;
         const int blocksY = (d.tilesY + 7) / 8;
         if (!persistentForm) {  // tiles of the chosen shape
             const int tw = 1 << twLog, th = 64 >> twLog;
@@ -383,9 +386,9 @@ int plan_views(const svo_view *views, int nviews, const svo_batch_opts *opts, in
     plan.slots = lds_slots(maxDepth, plan.reg);
     plan.wide = wide;
     plan.lod = lod;
-    const size_t ldsPerWave = size_t(plan.slots) * 64 * ((wide ? 8 : 4) + sizeof(float));
-    plan.ldsPerWave = ldsPerWave;
-    plan.ldsPerBlock = ldsPerWave * 4;
+    plan.levels = maxLevels;
+    plan.ldsPerWave = wide ? path_bytes<uint64_t>(maxLevels) : path_bytes<uint32_t>(maxLevels);
+    plan.ldsPerBlock = size_t(plan.slots) * 64 * ((wide ? 8 : 4) + sizeof(float)) * 4;
     const int form = opts ? opts->form : SVO_BATCH_GRID;
     if (form != SVO_BATCH_GRID && form != SVO_BATCH_PERSISTENT) return fail(SVO_ERR_INVALID, "unknown batch form");
     plan.persistent = form == SVO_BATCH_PERSISTENT;
@@ -423,44 +426,20 @@ void launch_batch(const LaunchPlan &p, const ViewDesc *dViews, const uint64_t *d
 }
 
 // Grid form: the tiles in launches of at most 2^31 - 1 workgroups.
-template <int Reg>
+template <bool Lod, typename Addr>
 void launch_tiles(const LaunchPlan &p, const ViewDesc *dViews, const uint64_t *dTileBase, hipStream_t s) {
     const uint64_t maxGrid = 0x7FFFFFFFull;
-    const TileOrder none{};
-    for (uint64_t first = 0; first < p.tiles; first += maxGrid) {
-        const dim3 grid(unsigned(std::min(maxGrid, p.tiles - first)));
-        if (!p.wide && !p.lod)
-            hipLaunchKernelGGL((tiles_kernel<false, uint32_t, Reg>), grid, dim3(64), p.ldsPerWave, s, dViews,
-                               dTileBase, p.nviews, first, p.slots, p.twLog, none);
-        else if (!p.wide)
-            hipLaunchKernelGGL((tiles_kernel<true, uint32_t, Reg>), grid, dim3(64), p.ldsPerWave, s, dViews,
-                               dTileBase, p.nviews, first, p.slots, p.twLog, none);
-        else if (!p.lod)
-            hipLaunchKernelGGL((tiles_kernel<false, uint64_t, Reg>), grid, dim3(64), p.ldsPerWave, s, dViews,
-                               dTileBase, p.nviews, first, p.slots, p.twLog, none);
-        else
-            hipLaunchKernelGGL((tiles_kernel<true, uint64_t, Reg>), grid, dim3(64), p.ldsPerWave, s, dViews,
-                               dTileBase, p.nviews, first, p.slots, p.twLog, none);
-    }
+    for (uint64_t first = 0; first < p.tiles; first += maxGrid)
+        hipLaunchKernelGGL((tiles_kernel<Lod, Addr>), dim3(unsigned(std::min(maxGrid, p.tiles - first))), dim3(64),
+                           p.ldsPerWave, s, dViews, dTileBase, p.nviews, first, p.levels, p.twLog, TileOrder{});
 }
 
 // Grid form in a tile plan's order: one launch (the plan holds at most 2^31 - 1 tiles).
-template <int Reg>
+template <bool Lod, typename Addr>
 void launch_tiles_planned(const LaunchPlan &p, const ViewDesc *dViews, const uint64_t *dTileBase, const TileOrder &o,
                           hipStream_t s) {
-    const dim3 grid(unsigned(p.tiles));
-    if (!p.wide && !p.lod)
-        hipLaunchKernelGGL((tiles_kernel<false, uint32_t, Reg, true>), grid, dim3(64), p.ldsPerWave, s, dViews,
-                           dTileBase, p.nviews, uint64_t(0), p.slots, p.twLog, o);
-    else if (!p.wide)
-        hipLaunchKernelGGL((tiles_kernel<true, uint32_t, Reg, true>), grid, dim3(64), p.ldsPerWave, s, dViews,
-                           dTileBase, p.nviews, uint64_t(0), p.slots, p.twLog, o);
-    else if (!p.lod)
-        hipLaunchKernelGGL((tiles_kernel<false, uint64_t, Reg, true>), grid, dim3(64), p.ldsPerWave, s, dViews,
-                           dTileBase, p.nviews, uint64_t(0), p.slots, p.twLog, o);
-    else
-        hipLaunchKernelGGL((tiles_kernel<true, uint64_t, Reg, true>), grid, dim3(64), p.ldsPerWave, s, dViews,
-                           dTileBase, p.nviews, uint64_t(0), p.slots, p.twLog, o);
+    hipLaunchKernelGGL((tiles_kernel<Lod, Addr, true>), dim3(unsigned(p.tiles)), dim3(64), p.ldsPerWave, s, dViews,
+                       dTileBase, p.nviews, uint64_t(0), p.levels, p.twLog, o);
 }
 
 }  // namespace
@@ -468,8 +447,10 @@ void launch_tiles_planned(const LaunchPlan &p, const ViewDesc *dViews, const uin
 void launch_plan(const LaunchPlan &p, const ViewDesc *dViews, const uint64_t *dTileBase, uint32_t *dCounters,
                  hipStream_t s) {
     if (!p.persistent) {
-        if (p.reg == 3) launch_tiles<3>(p, dViews, dTileBase, s);
-        else launch_tiles<1>(p, dViews, dTileBase, s);
+        if (!p.wide && !p.lod) launch_tiles<false, uint32_t>(p, dViews, dTileBase, s);
+        else if (!p.wide) launch_tiles<true, uint32_t>(p, dViews, dTileBase, s);
+        else if (!p.lod) launch_tiles<false, uint64_t>(p, dViews, dTileBase, s);
+        else launch_tiles<true, uint64_t>(p, dViews, dTileBase, s);
         return;
     }
     hipLaunchKernelGGL(zero_counters_kernel, dim3(1), dim3(64), 0, s, dCounters);
@@ -542,8 +523,10 @@ int render_batch_planned(svo_renderer *rd, const svo_view *views, int nviews, co
     HIP_TRY(hipMemcpyAsync(rd->dTileBase, rd->hTileBase, sizeof(uint64_t) * (nviews + 1), hipMemcpyHostToDevice, s));
     HIP_TRY(hipEventRecord(rd->staged, s));
     const TileOrder o = next_order(*tp);
-    if (plan.reg == 3) launch_tiles_planned<3>(plan, rd->dViews, rd->dTileBase, o, s);
-    else launch_tiles_planned<1>(plan, rd->dViews, rd->dTileBase, o, s);
+    if (!plan.wide && !plan.lod) launch_tiles_planned<false, uint32_t>(plan, rd->dViews, rd->dTileBase, o, s);
+    else if (!plan.wide) launch_tiles_planned<true, uint32_t>(plan, rd->dViews, rd->dTileBase, o, s);
+    else if (!plan.lod) launch_tiles_planned<false, uint64_t>(plan, rd->dViews, rd->dTileBase, o, s);
+    else launch_tiles_planned<true, uint64_t>(plan, rd->dViews, rd->dTileBase, o, s);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipEventRecord(rd->done, s));
     tp->renders++;

@@ -80,6 +80,7 @@ struct svo_octree {
     svo::WordVec words;           // Laine-Karras word array (src/VoxelOctree.hpp:40-41)
     float center[3] = {0, 0, 0};  // VoxelOctree::_center
     int depth = 0;                // descriptor levels + 1
+    int levels = 0;               // descriptor levels, childless descriptors included (at most depth)
     int device = -1;              // device holding `dwords`
     uint32_t *dwords = nullptr;   // device copy of `words`
     svo_build_stats build{};      // counters of the GPU build that made this tree (zeros otherwise)
@@ -128,7 +129,9 @@ void oct_encode(const svo_octree &h, std::vector<uint8_t> &out);
 // returns its depth (descriptor levels + 1), -1 if malformed (a reference
 // out of the array, a non-leaf slot with two parents, too deep), or -2 if
 // the check's one-bit-per-word bitmap cannot be allocated.
-int octree_validate(const uint32_t *words, uint64_t n);
+// *levels (may be null) receives the levels of descriptors, childless ones
+// included.
+int octree_validate(const uint32_t *words, uint64_t n, int *levels = nullptr);
 
 // ---- camera (camera.cpp) ----
 void orbit_camera(float pitch, float yaw, float radius, const float center[3], svo_camera &cam);
@@ -137,6 +140,15 @@ void orbit_camera(float pitch, float yaw, float radius, const float center[3], s
 bool camera_ok(const svo_camera &cam);
 
 // ---- device (raymarch.hip) ----
+// What a launch of one wave per workgroup that walks `h` needs: its levels,
+// 64-bit addresses for trees whose bytes do not fit 32-bit ones, and the LDS
+// of a wave's path stack.
+struct PathLaunch {
+    int levels;
+    bool wide;
+    size_t lds;
+};
+PathLaunch path_launch(const svo_octree &h);
 int ensure_device(svo_octree &h);
 void release_device(svo_octree &h);
 int raymarch_device(svo_octree &h, int64_t n, const float *o, const float *d, const float *rs,

@@ -34,7 +34,8 @@ struct LaunchPlan {
     int nviews = 0;
     uint64_t tiles = 0;
     int slots = 1;
-    int reg = 1;  // stack entries held in registers
+    int reg = 1;  // persistent form: stack entries held in registers
+    int levels = 1;  // grid form: path entries of a wave's stack
     bool wide = false, lod = false;
     size_t ldsPerBlock = 0;
     unsigned grid = 0;

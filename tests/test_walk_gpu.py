@@ -1,0 +1,71 @@
+"""The whole-ray walk's launch paths against the oracle at their edges: node
+forms and depths of the path stack, ray counts around a wave, finite and
+non-finite rays in one wave, level-of-detail cut-offs, trees at the end of
+the 32-bit byte addresses. Bit-exact."""
+import os
+
+import numpy as np
+import pytest
+
+import oracle_py as orc
+from test_format import relocated
+from walk_trees import mixed_tree
+
+pytestmark = pytest.mark.gpu
+
+
+def _same(mine, ref, what):
+    for k in ("hit", "normal", "leaf"):
+        assert np.array_equal(mine[k], ref[k]), (what, k)
+    assert np.array_equal(mine["t"].view(np.uint32), ref["t"].view(np.uint32)), what
+
+
+def _rays(n, seed):
+    rng = np.random.default_rng(seed)
+    o = rng.uniform(0.6, 2.4, (n, 3)).astype(np.float32)
+    d = (rng.uniform(1.1, 1.9, (n, 3)) - o).astype(np.float32)
+    return o, d, rng
+
+
+@pytest.mark.parametrize("levels", [1, 2, 3, 9, 10, 13, 14, 22, 23])
+def test_mixed_trees_match_oracle(svo, levels):
+    words = mixed_tree(levels, levels)
+    tree = svo.VoxelOctree.from_words(words, np.full(3, 0.5, np.float32))
+    print(f"[gpu] walk: mixed tree of {levels} levels, {len(words)} words", flush=True)
+    for n in (1, 63, 64, 65, 1000):
+        o, d, rng = _rays(n, 100 * levels + n)
+        _same(tree.raymarch_batch(o, d, 0.0), orc.raymarch(words, o, d, 0.0), ("no cut-off", n))
+        rs = rng.uniform(0.0, 0.1, n).astype(np.float32)
+        _same(tree.raymarch_batch(o, d, rs), orc.raymarch(words, o, d, rs), ("cut-off", n))
+        # non-finite and extreme rays between ordinary ones
+        d[::7, 0] = np.inf
+        d[::5, 1] = 0.0
+        o[::9, 2] = 3e30
+        d[1::11] *= np.float32(1e-30)
+        _same(tree.raymarch_batch(o, d, rs), orc.raymarch(words, o, d, rs), ("mixed rays", n))
+    cam = tree.orbit_camera(25.0, 40.0, 1.0)
+    tf, pos = np.frombuffer(cam.tform, np.float32), np.frombuffer(cam.pos, np.float32)
+    w, h = 93, 61
+    ref = orc.raymarch(words, pos[None, :], orc.primary_dirs(tf, w, h), 0.0)
+    _same(tree.render_primary(cam, w, h), ref, "primary")
+    rgba, depth = tree.render_frame(cam, 96, 64, 16, 1)
+    ref_rgba, ref_depth = orc.render_frame(words, tf, np.full(3, 0.5, np.float32), 96, 64, 16, 1)
+    assert np.array_equal(rgba, ref_rgba) and np.array_equal(depth.view(np.uint32), ref_depth.view(np.uint32))
+
+
+@pytest.mark.parametrize("short", [1, 0])
+def test_trees_at_the_end_of_32_bit_addresses(svo, golden, short):
+    """The dragon moved to the end of an array of 2^30 - short words: the last
+    size whose byte addresses fit 32 bits, and the first that takes 64."""
+    c, w = orc.read_oct(os.path.join(golden, "dragon.oct"))
+    base = (1 << 30) - short - len(w)
+    print(f"[gpu] walk: dragon at word {base}", flush=True)
+    big = svo.VoxelOctree.from_words(relocated(w, base), c)
+    assert big.word_count() == (1 << 30) - short
+    small = svo.VoxelOctree(os.path.join(golden, "dragon.oct"))
+    o, d, rng = _rays(5000, 3)
+    for rs in (0.0, rng.uniform(0.0, 0.05, 5000).astype(np.float32)):
+        mine, ref = big.raymarch_batch(o, d, rs), small.raymarch_batch(o, d, rs)
+        ref["leaf"] = np.where(ref["hit"] == 1, ref["leaf"] + np.uint64(base), ref["leaf"])
+        assert (ref["hit"] == 1).sum() > 10
+        _same(mine, ref, "rays")
