@@ -38,6 +38,7 @@ SVO_HD uint32_t bit0(uint32_t x) {
 #endif
 }
 
+SVO_HD int umin(int a, int b) { return a < b ? a : b; }
 // bit k of x
 SVO_HD uint32_t bit_at(uint32_t x, int k) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -326,17 +327,22 @@ SVO_HD int ray_step(Ray<Idx> &r, const uint32_t *__restrict__ tree, const Stack<
 // A pass takes an advance (or pop) where the cell cannot be entered and then,
 // in the same pass, the descent into the cell it reached where that can be
 // entered. A pop reads its node from LDS, so a pass waits for the tree's
-// memory once, for the descriptor it descended into.
+// memory once, for the descriptor it descended into (and its far word, which
+// travels with it). The next cell and its corner times are computed while that
+// read is under way and carried to the next pass.
 //
 // What bounds it: while all wave slots are busy VALU issue and the waits for
-// descriptors about equally (of the batch launch's wave-cycles 26% issue, 28%
-// wait to issue, 45% wait for memory; a wave executes nearly every pass's
-// advance and descent, 41 of 64 lanes active on average); at a launch's end
-// the dependent descriptor reads of the slowest tile. Against one step per
-// pass through ray_step (2048^3 mesh octree, 1920x1080, outputs equal): 3,752
-// -> 2,919 VALU instructions per wave and 8 views in one launch 1,391 ->
-// 1,112 us; one planned view 247 -> 210 us; 3840x2160 with shadows over an
-// 8192^3 terrain 1,515 -> 1,192 us; 1,021 rays 70 -> 39 us.
+// descriptors about equally (a wave executes nearly every pass's advance and
+// descent, 41 of 64 lanes active on average); at a launch's end the dependent
+// descriptor reads of the slowest tile. Against one step per pass through
+// ray_step (2048^3 mesh octree, 1920x1080, outputs equal): 8 views in one
+// launch 1,375 -> 965 us, one planned view 246 -> 157 us; 3840x2160 with
+// shadows over an 8192^3 terrain 1,515 -> 1,105 us. Of that, the corner times
+// carried over and computed behind the read (they were computed again at the
+// top of each pass, after the wait) gave 1,064 -> 978, 221 -> 191 and 1,267 ->
+// 1,179 us, the far word read beside its descriptor instead of after it 982 ->
+// 964, 181 -> 157 and 1,182 -> 1,104 us. A second advance per pass was slower
+// (982 -> 1,046 us: fewer passes, but more of them executed for few lanes).
 
 // The nodes on a ray's path, one entry per scale of their children: a node's
 // child block (a byte address from the tree's first word whose low two bits
@@ -372,12 +378,15 @@ SVO_HD uint32_t tree_word(const uint32_t *__restrict__ tree, Addr byte) {
     return *reinterpret_cast<const uint32_t *>(reinterpret_cast<const char *>(tree) + byte);
 }
 
-// The child block of the node whose descriptor `d` lies at byte p.
+// The child block of the node whose descriptor `d` lies at byte p; farWord is
+// the word after it where that has been read (have).
 template <typename Addr>
-SVO_HD Addr child_block(const uint32_t *__restrict__ tree, Addr p, uint32_t d) {
+SVO_HD Addr child_block(const uint32_t *__restrict__ tree, Addr p, uint32_t d, bool have, uint32_t farWord) {
     Addr b = p + Addr(d >> 16);  // bits 31..18 are words: shifted to bytes above the two flag bits
-    if (d & 0x20000u)
-        b = p + Addr(((uint64_t(d >> 18) << 32) | tree_word<Addr>(tree, p + 4)) << 2) + Addr((d >> 16) & 3u);
+    if (d & 0x20000u) {
+        if (!have) farWord = tree_word<Addr>(tree, p + 4);
+        b = p + Addr(((uint64_t(d >> 18) << 32) | farWord) << 2) + Addr((d >> 16) & 3u);
+    }
     return b;
 }
 
@@ -390,25 +399,38 @@ struct WalkEnd {
     SVO_HD Addr leaf() const { return (block >> 2) + Addr(popc32(((masks >> 8) << slot) & 127u)); }
 };
 
+// Work between a load and its first use: SVO_ISSUED keeps the code after it
+// behind the load, SVO_HOLD makes its values exist where it stands (ahead of
+// a later use of the loaded value).
+#if defined(__HIP_DEVICE_COMPILE__)
+#define SVO_ISSUED() __builtin_amdgcn_sched_barrier(0)
+#define SVO_HOLD(...) asm volatile("" : __VA_ARGS__)
+#else
+#define SVO_ISSUED()
+#define SVO_HOLD(...)
+#endif
+
 // Walks one ray (r from ray_init) to its end: kMiss, kLeaf (tOut, end) or, with
 // Lod, kLod (tOut). With Count, *passes counts the passes.
 template <bool Lod, bool Count, typename Addr>
 SVO_HD int walk(const Ray<Addr> &r, const uint32_t *__restrict__ tree, const PathStack<Addr> &path, float &tOut,
                 WalkEnd<Addr> &end, uint32_t *passes = nullptr) {
-    const uint32_t oct = uint32_t(r.octantMask);
+    // a cell's mask bits are shifted by its slot + 16: valid in bit 31,
+    // non-leaf in bit 23, its earlier siblings' non-leaf bits in 22..16
+    const uint32_t oct = uint32_t(r.octantMask) | 16u;
     float px = r.posX, py = r.posY, pz = r.posZ, minT = r.minT, e = 0.5f;
     int scale = kMaxScale - 1;
     uint32_t cs = uint32_t(r.idx) ^ oct, m = r.current;
-    Addr block = child_block<Addr>(tree, 0, m);
+    Addr block = child_block<Addr>(tree, 0, m, false, 0);
     path.put(scale, block, m);
-    int code;
-    for (;;) {
+    float tx = px * r.dTx - r.bTx, ty = py * r.dTy - r.bTy, tz = pz * r.dTz - r.bTz;
+    float tc = fminf(tx, fminf(ty, tz));
+    bool out = false, stop;
+    do {
         if (Count) ++*passes;
-        float tx = px * r.dTx - r.bTx, ty = py * r.dTy - r.bTy, tz = pz * r.dTz - r.bTz;
-        float tc = fminf(tx, fminf(ty, tz));
         uint32_t w = m << cs;
-        bool in = int16_t(w) < 0 && minT <= tc;
-        if (Lod && int16_t(w) < 0 && minT > tc) {
+        bool in = int32_t(w) < 0 && minT <= tc;
+        if (Lod && int32_t(w) < 0 && minT > tc) {
             // the reference's cut-off asks for minT <= the parent's exit only
             const uint32_t up = ~1u << scale;
             const float qx = u2f(f2u(px) & up) * r.dTx - r.bTx, qy = u2f(f2u(py) & up) * r.dTy - r.bTy,
@@ -425,11 +447,9 @@ SVO_HD int walk(const Ray<Addr> &r, const uint32_t *__restrict__ tree, const Pat
             if (tz <= tc) pz -= e;
             minT = tc;
             const uint32_t diff = (f2u(px) ^ ox) | (f2u(py) ^ oy) | (f2u(pz) ^ oz);
-            if (diff >= (1u << kMaxScale)) {
-                code = kMiss;
-                break;
-            }
-            scale = 31 - __builtin_clz(diff);
+            out = diff >= (1u << kMaxScale);
+            // a ray that left the tree reads the root's entry and stops below
+            scale = umin(31 - __builtin_clz(diff | 1u), kMaxScale - 1);
             e = u2f(uint32_t(scale - kMaxScale + 127) << 23);
             path.get(scale, block, m);
             const uint32_t keep = ~0u << scale;
@@ -442,20 +462,24 @@ SVO_HD int walk(const Ray<Addr> &r, const uint32_t *__restrict__ tree, const Pat
             tz = pz * r.dTz - r.bTz;
             tc = fminf(tx, fminf(ty, tz));
             w = m << cs;
-            in = int16_t(w) < 0 && minT <= tc;
+            in = int32_t(w) < 0 && minT <= tc && !out;
         }
-        if (in) {
-            if (Lod && tc * r.rayScale >= e) {
-                tOut = tc;
-                return kLod;
-            }
-            if (!(w & 0x80u)) {
-                code = kLeaf;
-                break;
-            }
-            const uint32_t sib = uint32_t(popc32(w & 127u));
+        if (Lod && in && tc * r.rayScale >= e) {
+            tOut = tc;
+            return kLod;
+        }
+        const bool down = in && (w & 0x800000u);
+        stop = out || (in && !(w & 0x800000u));
+        if (down) {
+            const uint32_t sib = uint32_t(popc32((w >> 16) & 127u));
             const Addr p = ((Addr(sib) << ((uint32_t(block) & 1u) | 2u)) + block) & ~Addr(3);
+            // a slot of two words holds a far word as a rule: both reads travel
+            // together (device arrays have a word to spare after the last)
+            const bool twoWords = uint32_t(block) & 1u;
+            uint32_t farWord = 0;
             m = tree_word<Addr>(tree, p);
+            if (twoWords) farWord = tree_word<Addr>(tree, p + 4);
+            SVO_ISSUED();
             --scale;
             e *= 0.5f;
             const bool cx = e * r.dTx + tx > minT, cy = e * r.dTy + ty > minT, cz = e * r.dTz + tz > minT;
@@ -463,15 +487,21 @@ SVO_HD int walk(const Ray<Addr> &r, const uint32_t *__restrict__ tree, const Pat
             if (cy) py += e;
             if (cz) pz += e;
             cs = ((cx ? 1u : 0u) | (cy ? 2u : 0u) | (cz ? 4u : 0u)) ^ oct;
-            block = child_block<Addr>(tree, p, m);
+            tx = px * r.dTx - r.bTx;
+            ty = py * r.dTy - r.bTy;
+            tz = pz * r.dTz - r.bTz;
+            tc = fminf(tx, fminf(ty, tz));
+            SVO_HOLD("+v"(cs), "+v"(tx), "+v"(ty), "+v"(tz), "+v"(tc));
+            SVO_HOLD("+v"(m));
+            block = child_block<Addr>(tree, p, m, twoWords, farWord);
             path.put(scale, block, m);
         }
-    }
+    } while (!stop);
     tOut = minT;
     end.block = block;
     end.masks = m;
-    end.slot = cs;
-    return code;
+    end.slot = cs & 7u;
+    return out ? kMiss : kLeaf;
 }
 
 }  // namespace march

@@ -56,9 +56,10 @@ int main(int argc, char **argv) {
     std::ifstream f(argv[1], std::ios::binary);
     std::vector<uint32_t> w;
     f.seekg(0, std::ios::end);
-    w.resize(size_t(f.tellg()) / 4);
+    const size_t bytes = size_t(f.tellg());
+    w.resize(bytes / 4 + 1, 0xFFFFFFFFu);  // the spare word of device arrays
     f.seekg(0);
-    f.read(reinterpret_cast<char *>(w.data()), std::streamsize(w.size() * 4));
+    f.read(reinterpret_cast<char *>(w.data()), std::streamsize(bytes));
     const int levels = std::atoi(argv[2]);
     const long n = std::atol(argv[3]);
     std::mt19937 g(7);
