@@ -128,7 +128,8 @@ template <typename Addr, int N, bool Planned = false>
 __global__ void __launch_bounds__(64) fine_kernel(const uint32_t *__restrict__ tree, const FrameSet<N> set,
                                                   unsigned tilesPerFrame, int levels, TileOrder o) {
     extern __shared__ __align__(16) unsigned char lds[];
-    const int64_t g = Planned ? int64_t(ordered_tile(o, int(blockIdx.x), int(threadIdx.x))) : int64_t(blockIdx.x);
+    const int64_t g = Planned ? int64_t(ordered_tile(o, int(blockIdx.x), int(threadIdx.x)))
+                              : int64_t(run_tile(blockIdx.x, gridDim.x));
     const unsigned f = N == 1 ? 0u : unsigned(g / tilesPerFrame);
     const int64_t tile = g - int64_t(f) * tilesPerFrame;
     const FrameParams &p = set.p[f];

@@ -118,7 +118,7 @@ __global__ void __launch_bounds__(64) primary_kernel(const uint32_t *__restrict_
                                                      int levels, uint8_t *hit, uint32_t *nrm, float *tt,
                                                      uint64_t *lf) {
     extern __shared__ __align__(16) unsigned char lds[];
-    const int tile = int(blockIdx.x);
+    const int tile = int(run_tile(blockIdx.x, gridDim.x));
     const int lane = threadIdx.x;
     const int x = (tile % p.tilesX) * 8 + (lane & 7);
     const int y = (tile / p.tilesX) * 8 + (lane >> 3);
@@ -179,7 +179,7 @@ __global__ void __launch_bounds__(64) primary_shadow_kernel(const uint32_t *__re
                                                             uint8_t *__restrict__ shadow, TileOrder o) {
     extern __shared__ __align__(16) unsigned char lds[];
     const int lane = threadIdx.x;
-    const int tile = Planned ? ordered_tile(o, int(blockIdx.x), lane) : int(blockIdx.x);
+    const int tile = Planned ? ordered_tile(o, int(blockIdx.x), lane) : int(run_tile(blockIdx.x, gridDim.x));
     const int x = (tile % p.tilesX) * 8 + (lane & 7);
     const int y = (tile / p.tilesX) * 8 + (lane >> 3);
     uint32_t passes = 0;

@@ -193,7 +193,8 @@ __global__ void __launch_bounds__(64) tiles_kernel(const ViewDesc *__restrict__ 
                                                    int levels, int twLog, TileOrder o) {
     extern __shared__ __align__(16) unsigned char lds[];
     const int lane = threadIdx.x;
-    const uint64_t tile = Planned ? uint64_t(ordered_tile(o, int(blockIdx.x), lane)) : first + blockIdx.x;
+    const uint64_t tile = Planned ? uint64_t(ordered_tile(o, int(blockIdx.x), lane))
+                                  : first + run_tile(blockIdx.x, gridDim.x);
     const int v = view_of(tileBase, nviews, tile);
     const ViewDesc &vd = views[v];
     const uint64_t local = tile - tileBase[v];

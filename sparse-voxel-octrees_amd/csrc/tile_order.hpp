@@ -76,6 +76,20 @@ inline TileOrder next_order(const svo_tile_plan &plan) {
     return o;
 }
 
+// Raster order dealt to the XCDs in runs: workgroup b runs on XCD b % 8, and
+// of every 8 * kTileRun tiles each XCD takes kTileRun neighbours instead of
+// every eighth tile, so the octree lines neighbouring tiles share are fetched
+// into one L2 (a 1-to-1 map of [0, n); a remainder of less than a full round
+// keeps its order). 8 views of 1920x1080 in one launch 967 -> 946 us, 64 mixed
+// views 1,907 -> 1,859, 1280x720 73.4 -> 69.8; runs of 4 gave half of that,
+// runs of 8 to 64 the same.
+constexpr uint32_t kXcds = 8, kTileRun = 16;
+__device__ __forceinline__ uint32_t run_tile(uint32_t b, uint32_t n) {
+    constexpr uint32_t kRound = kXcds * kTileRun;
+    const uint32_t at = b % kRound, round = b - at;
+    return n - round >= kRound ? round + (at % kXcds) * kTileRun + at / kXcds : b;
+}
+
 __device__ __forceinline__ int cost_bucket(uint32_t c) { return min(kCostBuckets - 1, 31 - __builtin_clz(c | 1u)); }
 
 __device__ __forceinline__ size_t replica_counts(int set, int rep) {
@@ -90,7 +104,7 @@ __device__ __forceinline__ size_t replica_ids(const TileOrder &o, int set, int r
 // fills.
 __device__ __forceinline__ int ordered_tile(const TileOrder &o, int b, int lane) {
     if (b < kReplicas && lane < kCostBuckets) o.counts[replica_counts(o.clr, b) + lane] = 0u;
-    if (o.src < 0) return b;
+    if (o.src < 0) return int(run_tile(uint32_t(b), uint32_t(o.tiles)));
     const int rep = b % kReplicas, k = b / kReplicas;
     const uint32_t c = lane < kCostBuckets ? o.counts[replica_counts(o.src, rep) + (kCostBuckets - 1 - lane)] : 0u;
     uint32_t incl = c;  // inclusive prefix over lanes 0..lane

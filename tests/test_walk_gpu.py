@@ -69,3 +69,36 @@ def test_trees_at_the_end_of_32_bit_addresses(svo, golden, short):
         ref["leaf"] = np.where(ref["hit"] == 1, ref["leaf"] + np.uint64(base), ref["leaf"])
         assert (ref["hit"] == 1).sum() > 10
         _same(mine, ref, "rays")
+
+
+@pytest.mark.parametrize("tiles", [1, 127, 128, 129, 255, 256, 383])
+def test_every_tile_runs_once_around_the_run_length(svo, golden, tiles):
+    """Tile counts around a full round of the XCD runs (128): the plain, the
+    planned (first and second launch) and the batched launch equal the oracle."""
+    import torch
+    tree = svo.VoxelOctree(os.path.join(golden, "dragon.oct"))
+    w, h = 8 * tiles, 8
+    cam = tree.orbit_camera(10.0, 30.0, 1.0)
+    tf, pos = np.frombuffer(cam.tform, np.float32), np.frombuffer(cam.pos, np.float32)
+    ref = orc.raymarch(tree.words(), pos[None, :], orc.primary_dirs(tf, w, h), 0.0)
+    _same(tree.render_primary(cam, w, h), ref, "plain")
+    out = {k: torch.full((w * h,), 7, dtype=dt, device="cuda")
+           for k, dt in (("hit", torch.uint8), ("normal", torch.int32), ("t", torch.float32), ("leaf", torch.int64))}
+    ptr = {k: v.data_ptr() for k, v in out.items()}
+
+    def got():
+        torch.cuda.synchronize()
+        r = {"hit": out["hit"].cpu().numpy(), "normal": out["normal"].cpu().numpy().view(np.uint32),
+             "t": out["t"].cpu().numpy(), "leaf": out["leaf"].cpu().numpy().view(np.uint64)}
+        for v in out.values():
+            v.fill_(7)
+        torch.cuda.synchronize()
+        return r
+
+    plan = svo.svo.TilePlan(w, h)
+    for k in range(3):
+        plan.render_device(tree, cam, ptr["hit"], ptr["normal"], ptr["t"], ptr["leaf"])
+        _same(got(), ref, ("planned", k))
+    ren = svo.svo.Renderer(2)
+    ren.render_device([ren.view(tree, cam, w, h, **ptr)])
+    _same(got(), ref, "batch")
