@@ -38,7 +38,7 @@ SVO_HD uint32_t bit0(uint32_t x) {
 #endif
 }
 
-SVO_HD int umin(int a, int b) { return a < b ? a : b; }
+SVO_HD int umax(int a, int b) { return uint32_t(a) > uint32_t(b) ? a : b; }
 // bit k of x
 SVO_HD uint32_t bit_at(uint32_t x, int k) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -336,13 +336,16 @@ SVO_HD int ray_step(Ray<Idx> &r, const uint32_t *__restrict__ tree, const Stack<
 // descent, 41 of 64 lanes active on average); at a launch's end the dependent
 // descriptor reads of the slowest tile. Against one step per pass through
 // ray_step (2048^3 mesh octree, 1920x1080, outputs equal): 8 views in one
-// launch 1,375 -> 965 us, one planned view 246 -> 157 us; 3840x2160 with
-// shadows over an 8192^3 terrain 1,515 -> 1,105 us. Of that, the corner times
+// launch 1,375 -> 896 us, one planned view 246 -> 152 us; 3840x2160 with
+// shadows over an 8192^3 terrain 1,515 -> 1,030 us. Of that, the corner times
 // carried over and computed behind the read (they were computed again at the
 // top of each pass, after the wait) gave 1,064 -> 978, 221 -> 191 and 1,267 ->
 // 1,179 us, the far word read beside its descriptor instead of after it 982 ->
-// 964, 181 -> 157 and 1,182 -> 1,104 us. A second advance per pass was slower
-// (982 -> 1,046 us: fewer passes, but more of them executed for few lanes).
+// 964, 181 -> 157 and 1,182 -> 1,104 us, a far test only in two-word slots, one
+// loop exit (the outcome read off the position afterwards) and the values
+// pinned by SVO_HOLD 945 -> 896, 154 -> 152 and 1,087 -> 1,030 us. A second
+// advance per pass was slower (982 -> 1,046 us: fewer passes, but more of them
+// executed for few lanes).
 
 // The nodes on a ray's path, one entry per scale of their children: a node's
 // child block (a byte address from the tree's first word whose low two bits
@@ -378,16 +381,14 @@ SVO_HD uint32_t tree_word(const uint32_t *__restrict__ tree, Addr byte) {
     return *reinterpret_cast<const uint32_t *>(reinterpret_cast<const char *>(tree) + byte);
 }
 
-// The child block of the node whose descriptor `d` lies at byte p; farWord is
-// the word after it where that has been read (have).
+// The child block of the node whose descriptor `d` lies at byte p: bits 31..18
+// are words, shifted to bytes above the two flag bits; with the far flag they
+// are the high bits of a word offset whose low 32 bits are farWord.
 template <typename Addr>
-SVO_HD Addr child_block(const uint32_t *__restrict__ tree, Addr p, uint32_t d, bool have, uint32_t farWord) {
-    Addr b = p + Addr(d >> 16);  // bits 31..18 are words: shifted to bytes above the two flag bits
-    if (d & 0x20000u) {
-        if (!have) farWord = tree_word<Addr>(tree, p + 4);
-        b = p + Addr(((uint64_t(d >> 18) << 32) | farWord) << 2) + Addr((d >> 16) & 3u);
-    }
-    return b;
+SVO_HD Addr near_block(Addr p, uint32_t d) { return p + Addr(d >> 16); }
+template <typename Addr>
+SVO_HD Addr far_block(Addr p, uint32_t d, uint32_t farWord) {
+    return p + Addr(((uint64_t(d >> 18) << 32) | farWord) << 2) + Addr((d >> 16) & 3u);
 }
 
 // Where a walk ended: the cell's child slot in the node `block`/`masks`.
@@ -415,17 +416,21 @@ struct WalkEnd {
 template <bool Lod, bool Count, typename Addr>
 SVO_HD int walk(const Ray<Addr> &r, const uint32_t *__restrict__ tree, const PathStack<Addr> &path, float &tOut,
                 WalkEnd<Addr> &end, uint32_t *passes = nullptr) {
+    // only descriptors in two-word slots have far words (the others, which no
+    // builder writes, take the 64-bit walk: path_launch)
+    constexpr bool Tight = sizeof(Addr) == 4;
     // a cell's mask bits are shifted by its slot + 16: valid in bit 31,
     // non-leaf in bit 23, its earlier siblings' non-leaf bits in 22..16
     const uint32_t oct = uint32_t(r.octantMask) | 16u;
     float px = r.posX, py = r.posY, pz = r.posZ, minT = r.minT, e = 0.5f;
     int scale = kMaxScale - 1;
     uint32_t cs = uint32_t(r.idx) ^ oct, m = r.current;
-    Addr block = child_block<Addr>(tree, 0, m, false, 0);
+    Addr block = near_block<Addr>(0, m);
+    if (m & 0x20000u) block = far_block<Addr>(0, m, tree[1]);
     path.put(scale, block, m);
     float tx = px * r.dTx - r.bTx, ty = py * r.dTy - r.bTy, tz = pz * r.dTz - r.bTz;
     float tc = fminf(tx, fminf(ty, tz));
-    bool out = false, stop;
+    bool stop;
     do {
         if (Count) ++*passes;
         uint32_t w = m << cs;
@@ -446,10 +451,12 @@ SVO_HD int walk(const Ray<Addr> &r, const uint32_t *__restrict__ tree, const Pat
             if (ty <= tc) py -= e;
             if (tz <= tc) pz -= e;
             minT = tc;
+            SVO_HOLD("+v"(minT));
             const uint32_t diff = (f2u(px) ^ ox) | (f2u(py) ^ oy) | (f2u(pz) ^ oz);
-            out = diff >= (1u << kMaxScale);
+            const bool out = diff >= (1u << kMaxScale);
             // a ray that left the tree reads the root's entry and stops below
-            scale = umin(31 - __builtin_clz(diff | 1u), kMaxScale - 1);
+            scale = 31 - umax(__builtin_clz(diff), 32 - kMaxScale);
+            SVO_HOLD("+v"(scale));
             e = u2f(uint32_t(scale - kMaxScale + 127) << 23);
             path.get(scale, block, m);
             const uint32_t keep = ~0u << scale;
@@ -462,23 +469,29 @@ SVO_HD int walk(const Ray<Addr> &r, const uint32_t *__restrict__ tree, const Pat
             tz = pz * r.dTz - r.bTz;
             tc = fminf(tx, fminf(ty, tz));
             w = m << cs;
-            in = int32_t(w) < 0 && minT <= tc && !out;
+            in = int32_t(w) < 0 && minT <= tc;
+            if (out) {  // stops like a leaf
+                in = true;
+                w = 0;
+            }
         }
-        if (Lod && in && tc * r.rayScale >= e) {
+        if (Lod && in && w && tc * r.rayScale >= e) {
             tOut = tc;
             return kLod;
         }
         const bool down = in && (w & 0x800000u);
-        stop = out || (in && !(w & 0x800000u));
+        stop = in && !down;
         if (down) {
             const uint32_t sib = uint32_t(popc32((w >> 16) & 127u));
-            const Addr p = ((Addr(sib) << ((uint32_t(block) & 1u) | 2u)) + block) & ~Addr(3);
-            // a slot of two words holds a far word as a rule: both reads travel
-            // together (device arrays have a word to spare after the last)
-            const bool twoWords = uint32_t(block) & 1u;
-            uint32_t farWord = 0;
+            uint32_t width = (uint32_t(block) & 1u) | 2u;  // log2 of a slot's bytes
+            SVO_HOLD("+v"(width));
+            const Addr p = ((Addr(sib) << width) + block) & ~Addr(3);
+            // a two-word slot's far word travels with its descriptor (device
+            // arrays have a word to spare after the last)
+            const bool two = width == 3;
+            uint32_t farWord;
             m = tree_word<Addr>(tree, p);
-            if (twoWords) farWord = tree_word<Addr>(tree, p + 4);
+            if (two) farWord = tree_word<Addr>(tree, p + 4);
             SVO_ISSUED();
             --scale;
             e *= 0.5f;
@@ -493,7 +506,15 @@ SVO_HD int walk(const Ray<Addr> &r, const uint32_t *__restrict__ tree, const Pat
             tc = fminf(tx, fminf(ty, tz));
             SVO_HOLD("+v"(cs), "+v"(tx), "+v"(ty), "+v"(tz), "+v"(tc));
             SVO_HOLD("+v"(m));
-            block = child_block<Addr>(tree, p, m, twoWords, farWord);
+            block = near_block<Addr>(p, m);
+            if (Tight) {
+                if (two) {
+                    SVO_HOLD("+v"(farWord));  // not shifted before the wait
+                    if (m & 0x20000u) block = far_block<Addr>(p, m, farWord);
+                }
+            } else if (m & 0x20000u) {
+                block = far_block<Addr>(p, m, two ? farWord : tree_word<Addr>(tree, p + 4));
+            }
             path.put(scale, block, m);
         }
     } while (!stop);
@@ -501,7 +522,8 @@ SVO_HD int walk(const Ray<Addr> &r, const uint32_t *__restrict__ tree, const Pat
     end.block = block;
     end.masks = m;
     end.slot = cs & 7u;
-    return out ? kMiss : kLeaf;
+    // outside the tree a coordinate is below 1 (bit 23 of its float clear)
+    return (f2u(px) & f2u(py) & f2u(pz) & (1u << kMaxScale)) ? kLeaf : kMiss;
 }
 
 }  // namespace march

@@ -44,9 +44,10 @@ struct Item {
 // pointers only point forward, so with that rule the check visits each word
 // at most once. With `frontier`, nodes at level `split` are handed out
 // instead of descended into.
-// *levels receives the levels of descriptors visited, childless ones included.
+// levels is raised to the levels of descriptors visited, childless ones
+// included; tight is cleared by a far word in a one-word slot.
 int validate_from(const uint32_t *w, uint64_t n, Item root, int split, std::vector<Item> *frontier, uint64_t *seen,
-                  int &levels) {
+                  int &levels, bool &tight) {
     std::vector<Item> stack;
     stack.push_back(root);
     int depth = 0;
@@ -80,6 +81,7 @@ int validate_from(const uint32_t *w, uint64_t n, Item root, int split, std::vect
                 uint64_t coff = cw >> 18;
                 if (cw & 0x20000u) {
                     if (slot + 1 >= n) return -1;
+                    if (per == 1) tight = false;
                     coff = (coff << 32) | w[slot + 1];
                 }
                 if (coff == 0) return -1;  // a node cannot be its own child block
@@ -101,7 +103,7 @@ int validate_from(const uint32_t *w, uint64_t n, Item root, int split, std::vect
 // (levels of descriptors + 1), -1 for a malformed tree or -2 when the check's
 // bitmap (one bit per word) cannot be allocated. Subtrees below level 3 are
 // checked on all host threads.
-int octree_validate(const uint32_t *w, uint64_t n, int *levelsOut) {
+int octree_validate(const uint32_t *w, uint64_t n, int *levelsOut, bool *tightOut) {
     if (n == 0) return -1;
     // the root's child offset, far form included: the traversal reads it like
     // any other descriptor's (src/VoxelOctree.cpp:276-280)
@@ -119,18 +121,22 @@ int octree_validate(const uint32_t *w, uint64_t n, int *levelsOut) {
     std::vector<Item> frontier;
     const int split = 3;
     int levels = 1;
-    int depth = validate_from(w, n, {0, rootOff, 0}, split, &frontier, seen, levels);
+    bool tight = true;
+    int depth = validate_from(w, n, {0, rootOff, 0}, split, &frontier, seen, levels, tight);
     if (depth < 0) return -1;
     depth = std::max(depth, 1);
     if (levelsOut) *levelsOut = levels;
+    if (tightOut) *tightOut = tight;
     if (frontier.empty()) return depth;
     std::atomic<size_t> next{0};
     std::atomic<int> worst{depth}, most{levels};
-    std::atomic<bool> bad{false};
+    std::atomic<bool> bad{false}, loose{!tight};
     auto worker = [&]() {
         for (size_t i; !bad.load() && (i = next.fetch_add(1)) < frontier.size();) {
             int lv = 1;
-            int d = validate_from(w, n, frontier[i], split, nullptr, seen, lv);
+            bool tg = true;
+            int d = validate_from(w, n, frontier[i], split, nullptr, seen, lv, tg);
+            if (!tg) loose.store(true);
             if (d < 0) {
                 bad.store(true);
                 return;
@@ -152,6 +158,7 @@ int octree_validate(const uint32_t *w, uint64_t n, int *levelsOut) {
     worker();
     for (std::thread &t : pool) t.join();
     if (levelsOut) *levelsOut = most.load();
+    if (tightOut) *tightOut = !loose.load();
     return bad.load() ? -1 : worst.load();
 }
 

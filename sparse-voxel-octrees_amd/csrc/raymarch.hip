@@ -242,7 +242,7 @@ int raymarch_one(const svo_octree &h, const float o[3], const float d[3], float 
 PathLaunch path_launch(const svo_octree &h) {
     PathLaunch L;
     L.levels = h.levels;
-    L.wide = h.words.size() >= (uint64_t(1) << 30);
+    L.wide = h.words.size() >= (uint64_t(1) << 30) || !h.tight;
     L.lds = L.wide ? path_bytes<uint64_t>(L.levels) : path_bytes<uint32_t>(L.levels);
     return L;
 }

@@ -29,7 +29,7 @@ void clear_error() { g_error.clear(); }
 // with leaves itself, after its scatter checked every node's slot and child
 // block against the array; its other trees are walked like the rest.
 static int finish_handle(std::unique_ptr<svo_octree> &h, svo_octree **out) {
-    int depth = h->depth > 0 ? h->depth : octree_validate(h->words.data(), h->words.size(), &h->levels);
+    int depth = h->depth > 0 ? h->depth : octree_validate(h->words.data(), h->words.size(), &h->levels, &h->tight);
     if (depth < 0) {
         release_device(*h);
         if (depth == -2) return fail(SVO_ERR_NOMEM, "out of host memory (octree check)");

@@ -81,6 +81,7 @@ struct svo_octree {
     float center[3] = {0, 0, 0};  // VoxelOctree::_center
     int depth = 0;                // descriptor levels + 1
     int levels = 0;               // descriptor levels, childless descriptors included (at most depth)
+    bool tight = true;            // only descriptors in two-word slots (and the root) have far words
     int device = -1;              // device holding `dwords`
     uint32_t *dwords = nullptr;   // device copy of `words`
     svo_build_stats build{};      // counters of the GPU build that made this tree (zeros otherwise)
@@ -129,9 +130,10 @@ void oct_encode(const svo_octree &h, std::vector<uint8_t> &out);
 // returns its depth (descriptor levels + 1), -1 if malformed (a reference
 // out of the array, a non-leaf slot with two parents, too deep), or -2 if
 // the check's one-bit-per-word bitmap cannot be allocated.
-// *levels (may be null) receives the levels of descriptors, childless ones
-// included.
-int octree_validate(const uint32_t *words, uint64_t n, int *levels = nullptr);
+// *levels receives the levels of descriptors, childless ones included, *tight
+// whether only descriptors in two-word slots (and the root) have far words
+// (either may be null).
+int octree_validate(const uint32_t *words, uint64_t n, int *levels = nullptr, bool *tight = nullptr);
 
 // ---- camera (camera.cpp) ----
 void orbit_camera(float pitch, float yaw, float radius, const float center[3], svo_camera &cam);
@@ -141,8 +143,9 @@ bool camera_ok(const svo_camera &cam);
 
 // ---- device (raymarch.hip) ----
 // What a launch of one wave per workgroup that walks `h` needs: its levels,
-// 64-bit addresses for trees whose bytes do not fit 32-bit ones, and the LDS
-// of a wave's path stack.
+// whether it takes the 64-bit walk (trees whose bytes do not fit 32-bit
+// addresses, and trees with far words in one-word slots, which the 32-bit walk
+// does not look for), and the LDS of a wave's path stack.
 struct PathLaunch {
     int levels;
     bool wide;

@@ -20,16 +20,17 @@ def walk_test(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("tree", ["dragon", "mixed1", "mixed2", "mixed3", "mixed10", "mixed22", "mixed23"])
+@pytest.mark.parametrize("tree", ["dragon", "mixed1", "mixed2", "mixed3", "mixed10", "mixed22", "mixed23",
+                                  "loose3", "loose10"])
 def test_walk_equals_the_reference_loop(walk_test, golden, tmp_path, tree):
     if tree == "dragon":
         _, words = orc.read_oct(os.path.join(golden, "dragon.oct"))
         levels = 8
     else:
         levels = int(tree[5:])
-        words = mixed_tree(levels, levels)
+        words = mixed_tree(levels, levels, loose=tree.startswith("loose"))
     path = str(tmp_path / "words.bin")
     np.ascontiguousarray(words, np.uint32).tofile(path)
-    r = subprocess.run([walk_test, path, str(levels), "20000"], capture_output=True, text=True, timeout=300)
+    r = subprocess.run([walk_test, path, str(levels), "20000"] + (["loose"] if tree.startswith("loose") else []), capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stdout + r.stderr
     assert r.stdout.startswith("ok ")

@@ -27,9 +27,9 @@ def _rays(n, seed):
     return o, d, rng
 
 
-@pytest.mark.parametrize("levels", [1, 2, 3, 9, 10, 13, 14, 22, 23])
-def test_mixed_trees_match_oracle(svo, levels):
-    words = mixed_tree(levels, levels)
+@pytest.mark.parametrize("levels,loose", [(n, False) for n in (1, 2, 3, 9, 10, 13, 14, 22, 23)] + [(3, True), (10, True)])
+def test_mixed_trees_match_oracle(svo, levels, loose):
+    words = mixed_tree(levels, levels, loose=loose)
     tree = svo.VoxelOctree.from_words(words, np.full(3, 0.5, np.float32))
     print(f"[gpu] walk: mixed tree of {levels} levels, {len(words)} words", flush=True)
     for n in (1, 63, 64, 65, 1000):

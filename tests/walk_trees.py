@@ -3,12 +3,13 @@ allows the traversal to meet, at up to the full 23 levels."""
 import numpy as np
 
 
-def mixed_tree(seed, levels, fanout=2.2):
+def mixed_tree(seed, levels, fanout=2.2, loose=False):
     """Random tree with leaves, childless descriptors and far (two-word) child
     slots at every level; `levels` descriptor levels. Masks are as the
     reference writes them (a node's children are all descriptors or all
     leaves). One path always reaches the last level, whose descriptor there is
-    childless when the seed is odd."""
+    childless when the seed is odd. loose: some one-word child blocks are
+    followed by a word that their last child uses as its far word."""
     rng = np.random.default_rng(seed)
 
     def node(level, spine):
@@ -30,7 +31,7 @@ def mixed_tree(seed, levels, fanout=2.2):
         if spine or not valid:
             valid |= 1 << keep
         kids = [node(level + 1, spine and c == keep) for c in range(8) if valid >> c & 1]
-        return (valid, kids, bool(rng.random() < 0.4) or size(kids) > 0x3000)
+        return (valid, kids, bool(rng.random() < 0.4) or size(kids) > 0x2000)
 
     def size(kids):
         return sum(2 + (bin(k[0]).count("1") if k[1] is None else size(k[1])) for k in kids)
@@ -53,9 +54,10 @@ def mixed_tree(seed, levels, fanout=2.2):
             words.extend(int(x) | 1 for x in rng.integers(0, 1 << 32, bin(valid).count("1")))
             return
         per = 2 if large else 1
-        words.extend([0] * (per * len(kids)))
+        spare = loose and not large and rng.random() < 0.5
+        words.extend([0] * (per * len(kids) + spare))
         for i, k in enumerate(kids):
-            emit(k, start + i * per, large)
+            emit(k, start + i * per, large or (spare and i == len(kids) - 1))
 
     root = node(0, True)
     words.append(0)
