@@ -48,6 +48,21 @@ SVO_HD uint32_t bit_at(uint32_t x, int k) {
 #endif
 }
 
+// All ones where a < b (finite), else 0: the sign of the difference, which is
+// zero only for equal values.
+SVO_HD uint32_t lt_bits(float a, float b) { return uint32_t(int32_t(f2u(a - b)) >> 31); }
+// Bitwise function of three words by its truth table (a = 0xF0, b = 0xCC, c = 0xAA).
+template <int Table>
+SVO_HD uint32_t bitop(uint32_t a, uint32_t b, uint32_t c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_bitop3_b32(a, b, c, Table);
+#else
+    uint32_t r = 0;
+    for (int k = 0; k < 8; ++k)
+        if (Table >> k & 1) r |= (k & 4 ? a : ~a) & (k & 2 ? b : ~b) & (k & 1 ? c : ~c);
+    return r;
+#endif
+}
 // invSqrt, src/Util.hpp:47-58
 SVO_HD float quake_rsqrt(float x) {
     float half = x * 0.5f;
@@ -336,8 +351,8 @@ SVO_HD int ray_step(Ray<Idx> &r, const uint32_t *__restrict__ tree, const Stack<
 // descent, 41 of 64 lanes active on average); at a launch's end the dependent
 // descriptor reads of the slowest tile. Against one step per pass through
 // ray_step (2048^3 mesh octree, 1920x1080, outputs equal): 8 views in one
-// launch 1,375 -> 896 us, one planned view 246 -> 152 us; 3840x2160 with
-// shadows over an 8192^3 terrain 1,515 -> 1,030 us. Of that, the corner times
+// launch 1,375 -> 858 us, one planned view 246 -> 146 us; 3840x2160 with
+// shadows over an 8192^3 terrain 1,515 -> 985 us. Of that, the corner times
 // carried over and computed behind the read (they were computed again at the
 // top of each pass, after the wait) gave 1,064 -> 978, 221 -> 191 and 1,267 ->
 // 1,179 us, the far word read beside its descriptor instead of after it 982 ->
@@ -346,6 +361,16 @@ SVO_HD int ray_step(Ray<Idx> &r, const uint32_t *__restrict__ tree, const Stack<
 // pinned by SVO_HOLD 945 -> 896, 154 -> 152 and 1,087 -> 1,030 us. A second
 // advance per pass was slower (982 -> 1,046 us: fewer passes, but more of them
 // executed for few lanes).
+//
+// The loop prefers instructions that issue two per four cycles on a SIMD
+// (measured on this card with all wave slots busy: f32 add, subtract, multiply,
+// and/or/xor, right shifts, u32 add and subtract, bitop3) over those that issue
+// one (compares, selects, min/max, left shifts, bit-field extracts, shift-adds,
+// anything with a scalar operand): a selection is a sign mask and an `and`
+// (lt_bits, bitop) where that takes no more instructions. 45 of the pass's 86
+// instructions were of the slower kind, 26 of 87 now: 893 -> 858, 151 -> 146
+// and 1,029 -> 985 us. Trading the position bits' three extracts for six
+// faster instructions gave nothing more.
 
 // The nodes on a ray's path, one entry per scale of their children: a node's
 // child block (a byte address from the tree's first word whose low two bits
@@ -434,7 +459,7 @@ SVO_HD int walk(const Ray<Addr> &r, const uint32_t *__restrict__ tree, const Pat
     do {
         if (Count) ++*passes;
         uint32_t w = m << cs;
-        bool in = int32_t(w) < 0 && minT <= tc;
+        bool in = int32_t(bitop<0x30>(w, f2u(tc - minT), 0u)) < 0;
         if (Lod && int32_t(w) < 0 && minT > tc) {
             // the reference's cut-off asks for minT <= the parent's exit only
             const uint32_t up = ~1u << scale;
@@ -447,12 +472,12 @@ SVO_HD int walk(const Ray<Addr> &r, const uint32_t *__restrict__ tree, const Pat
         }
         if (!in) {
             const uint32_t ox = f2u(px), oy = f2u(py), oz = f2u(pz);
-            if (tx <= tc) px -= e;
-            if (ty <= tc) py -= e;
-            if (tz <= tc) pz -= e;
+            px -= u2f(bitop<0x30>(f2u(e), lt_bits(tc, tx), 0u));  // e where the axis's corner time is the smallest
+            py -= u2f(bitop<0x30>(f2u(e), lt_bits(tc, ty), 0u));
+            pz -= u2f(bitop<0x30>(f2u(e), lt_bits(tc, tz), 0u));
             minT = tc;
             SVO_HOLD("+v"(minT));
-            const uint32_t diff = (f2u(px) ^ ox) | (f2u(py) ^ oy) | (f2u(pz) ^ oz);
+            const uint32_t diff = bitop<0xBE>(f2u(pz), oz, bitop<0xBE>(f2u(py), oy, f2u(px) ^ ox));
             const bool out = diff >= (1u << kMaxScale);
             // a ray that left the tree reads the root's entry and stops below
             scale = 31 - umax(__builtin_clz(diff), 32 - kMaxScale);
@@ -469,7 +494,7 @@ SVO_HD int walk(const Ray<Addr> &r, const uint32_t *__restrict__ tree, const Pat
             tz = pz * r.dTz - r.bTz;
             tc = fminf(tx, fminf(ty, tz));
             w = m << cs;
-            in = int32_t(w) < 0 && minT <= tc;
+            in = int32_t(bitop<0x30>(w, f2u(tc - minT), 0u)) < 0;
             if (out) {  // stops like a leaf
                 in = true;
                 w = 0;
@@ -482,8 +507,8 @@ SVO_HD int walk(const Ray<Addr> &r, const uint32_t *__restrict__ tree, const Pat
         const bool down = in && (w & 0x800000u);
         stop = in && !down;
         if (down) {
-            const uint32_t sib = uint32_t(popc32((w >> 16) & 127u));
-            uint32_t width = (uint32_t(block) & 1u) | 2u;  // log2 of a slot's bytes
+            const uint32_t sib = uint32_t(popc32(w & 0x7F0000u));
+            uint32_t width = bitop<0xEA>(uint32_t(block), 1u, 2u);  // log2 of a slot's bytes
             SVO_HOLD("+v"(width));
             const Addr p = ((Addr(sib) << width) + block) & ~Addr(3);
             // a two-word slot's far word travels with its descriptor (device
@@ -495,11 +520,12 @@ SVO_HD int walk(const Ray<Addr> &r, const uint32_t *__restrict__ tree, const Pat
             SVO_ISSUED();
             --scale;
             e *= 0.5f;
-            const bool cx = e * r.dTx + tx > minT, cy = e * r.dTy + ty > minT, cz = e * r.dTz + tz > minT;
-            if (cx) px += e;
-            if (cy) py += e;
-            if (cz) pz += e;
-            cs = ((cx ? 1u : 0u) | (cy ? 2u : 0u) | (cz ? 4u : 0u)) ^ oct;
+            const uint32_t mx = lt_bits(minT, e * r.dTx + tx), my = lt_bits(minT, e * r.dTy + ty),
+                           mz = lt_bits(minT, e * r.dTz + tz);
+            px += u2f(bitop<0xC0>(f2u(e), mx, 0u));
+            py += u2f(bitop<0xC0>(f2u(e), my, 0u));
+            pz += u2f(bitop<0xC0>(f2u(e), mz, 0u));
+            cs = bitop<0x78>(bitop<0x78>(bitop<0x78>(oct, mx, 1u), my, 2u), mz, 4u);  // oct ^ (mx & 1) ^ ...
             tx = px * r.dTx - r.bTx;
             ty = py * r.dTy - r.bTy;
             tz = pz * r.dTz - r.bTz;
