@@ -59,6 +59,15 @@ using namespace dev;
 
 constexpr int kThreads = 256;
 
+// rocPRIM sorts arrays below this size by merging, two launches per doubling
+// above 1024 items (20 launches for the 480 K candidates of a 256^3 mesh);
+// from here up its radix passes (one per 8 key bits, three or so) are faster.
+// 256^3 mesh build 1.12 -> 1.03 ms, a 203x251x189 volume 2.18 -> 2.10 ms;
+// with the line at 2^12 or 2^14 a 64^3 mesh (30 K candidates) took 0.85
+// instead of 0.75 ms. The default line is 2^20.
+using SortConfig = rocprim::radix_sort_config<rocprim::default_config, rocprim::default_config, rocprim::default_config,
+                                              size_t(1) << 17>;
+
 inline unsigned grid_for(uint64_t n) { return unsigned((n + kThreads - 1) / kThreads); }
 
 // Device memory and stream of one build, kept between builds: a workspace
@@ -2426,10 +2435,10 @@ static int mesh_core(Arena &ar, float *dv, int64_t nverts, int has_normals, int3
     if (K) {
         size_t bytes = 0;
         const int endBit = 3 * g.depth + tribits;
-        HIP_TRY(rocprim::radix_sort_keys(nullptr, bytes, keys, keys2, K, tribits, endBit, st));
+        HIP_TRY(rocprim::radix_sort_keys<SortConfig>(nullptr, bytes, keys, keys2, K, tribits, endBit, st));
         uint8_t *tmp;
         if ((r = ar.alloc(tmp, bytes))) return r;
-        HIP_TRY(rocprim::radix_sort_keys(tmp, bytes, keys, keys2, K, tribits, endBit, st));
+        HIP_TRY(rocprim::radix_sort_keys<SortConfig>(tmp, bytes, keys, keys2, K, tribits, endBit, st));
         ar.release(tmp);
     }
     ar.release(keys);
@@ -2720,10 +2729,10 @@ int build_grid(const uint32_t *grid, int w, int h, int d, const svo_build_opts *
     ar.release(at);
     if (V) {
         size_t bytes = 0;
-        HIP_TRY(rocprim::radix_sort_pairs(nullptr, bytes, key, key2, word, word2, V, 0, 3 * g.depth, st));
+        HIP_TRY(rocprim::radix_sort_pairs<SortConfig>(nullptr, bytes, key, key2, word, word2, V, 0, 3 * g.depth, st));
         uint8_t *tmp;
         if ((r = ar.alloc(tmp, bytes))) return r;
-        HIP_TRY(rocprim::radix_sort_pairs(tmp, bytes, key, key2, word, word2, V, 0, 3 * g.depth, st));
+        HIP_TRY(rocprim::radix_sort_pairs<SortConfig>(tmp, bytes, key, key2, word, word2, V, 0, 3 * g.depth, st));
         ar.release(tmp);
     }
     uint32_t *blockFlags;
@@ -2782,10 +2791,10 @@ static int sdf_leaves(Arena &ar, const svo_sdf_primitive *prims, int count, int 
             if ((r = ar.alloc(k2, V)) || (r = ar.alloc(w2, V))) return r;
             if (V) {
                 size_t bytes = 0;
-                HIP_TRY(rocprim::radix_sort_pairs(nullptr, bytes, k, k2, w, w2, V, 0, 3 * log2i(n), st));
+                HIP_TRY(rocprim::radix_sort_pairs<SortConfig>(nullptr, bytes, k, k2, w, w2, V, 0, 3 * log2i(n), st));
                 uint8_t *tmp;
                 if ((r = ar.alloc(tmp, bytes))) return r;
-                HIP_TRY(rocprim::radix_sort_pairs(tmp, bytes, k, k2, w, w2, V, 0, 3 * log2i(n), st));
+                HIP_TRY(rocprim::radix_sort_pairs<SortConfig>(tmp, bytes, k, k2, w, w2, V, 0, 3 * log2i(n), st));
                 ar.release(tmp);
             }
             ar.release(k);
@@ -2843,10 +2852,10 @@ static int terrain_leaves(Arena &ar, int n, uint32_t seed, uint64_t *&key, uint3
     uint32_t *w2;
     if ((r = ar.alloc(k2, V)) || (r = ar.alloc(w2, V))) return r;
     size_t bytes = 0;
-    HIP_TRY(rocprim::radix_sort_keys(nullptr, bytes, k, k2, V, 0, 3 * log2i(n), st));
+    HIP_TRY(rocprim::radix_sort_keys<SortConfig>(nullptr, bytes, k, k2, V, 0, 3 * log2i(n), st));
     uint8_t *tmp;
     if ((r = ar.alloc(tmp, bytes))) return r;
-    HIP_TRY(rocprim::radix_sort_keys(tmp, bytes, k, k2, V, 0, 3 * log2i(n), st));
+    HIP_TRY(rocprim::radix_sort_keys<SortConfig>(tmp, bytes, k, k2, V, 0, 3 * log2i(n), st));
     ar.release(tmp);
     ar.release(k);
     if (V) hipLaunchKernelGGL(terrain_words_kernel, dim3(grid_for(V)), dim3(kThreads), 0, st, k2, V, n, colWord, w2);
