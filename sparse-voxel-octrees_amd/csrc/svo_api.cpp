@@ -24,6 +24,8 @@ int fail(int code, const std::string &msg) {
 
 void clear_error() { g_error.clear(); }
 
+std::string last_error() { return g_error; }
+
 // Trees from files and caller arrays are walked on the host (octree_validate)
 // before anything traverses them. The GPU builder sets the depth of a tree
 // with leaves itself, after its scatter checked every node's slot and child

@@ -98,6 +98,7 @@ namespace svo {
 // thread-local error message; returns `code` for convenient `return fail(...)`
 int fail(int code, const std::string &msg);
 void clear_error();
+std::string last_error();  // this thread's message
 
 // ---- .oct codec (lz4_oct.cpp) ----
 // Appends the LZ4 block encoding of src[pos, pos+len) to `out`, continuing the

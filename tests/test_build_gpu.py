@@ -487,3 +487,35 @@ def test_build_stats_are_consistent(svo, tmp_path):
     assert gs["triangles"] == 0 and gs["candidates"] == gs["leaves"] == orc.octree_stats(g.words())["leaves"]
     loaded = svo.VoxelOctree.from_words(words, t.center())
     assert loaded.build_stats()["words"] == 0 and loaded.build_stats()["peak_bytes"] == 0
+
+
+@pytest.mark.parametrize("nq", [0, 1, 40000])
+def test_large_meshes_checked_on_the_device(svo, golden, nq):
+    """A mesh above the size from which checks, bounds and face tables are made
+    on the device: triangles only (nq = 0), and triangles with some quads
+    first or between them, against the oracle's build; and each refusal."""
+    rng = np.random.default_rng(17)
+    n = 40000 - nq // 2
+    centre = rng.uniform(0.1, 0.9, (n, 3))
+    v = (centre[:, None, :] + rng.normal(scale=0.01, size=(n, 4, 3))).astype(np.float32).reshape(-1, 3)
+    counts = np.full(n, 3, np.int32)
+    counts[:1 if nq == 1 else 0] = 4
+    if nq > 1:
+        counts[rng.random(n) < 0.5] = 4
+    idx = np.concatenate([4 * f + np.arange(c) for f, c in enumerate(counts)]).astype(np.int32)
+    tab = np.zeros((len(v), 9), np.float32)
+    tab[:, :3], tab[:, 6:] = v, 255.0
+    print(f"[gpu] mesh of {len(v)} vertices and {n} faces, {int((counts == 4).sum())} quads", flush=True)
+    assert len(v) + n >= 1 << 16
+    t = svo.VoxelOctree.build_from_mesh(tab, False, counts, idx, 64, threads=8, memory_budget=1 << 30)
+    center, words, _ = orc.Mesh(tab, False, counts, idx).build(64, 8, 1 << 30)
+    assert np.array_equal(t.words(), words) and np.array_equal(t.center(), center)
+    for code, hurt in ((svo.svo.ERR_UNSUPPORTED, lambda a, c, i: a.__setitem__((len(a) - 1, 2), np.inf)),
+                       (svo.svo.ERR_FORMAT, lambda a, c, i: i.__setitem__(len(i) - 1, len(v))),
+                       (svo.svo.ERR_FORMAT, lambda a, c, i: i.__setitem__(7, -1)),
+                       (svo.svo.ERR_FORMAT, lambda a, c, i: c.__setitem__(5, -3))):
+        a, c, i = tab.copy(), counts.copy(), idx.copy()
+        hurt(a, c, i)
+        with pytest.raises(svo.SvoError) as e:
+            svo.VoxelOctree.build_from_mesh(a, False, c, i, 64, threads=8)
+        assert e.value.code == code
