@@ -519,3 +519,29 @@ def test_large_meshes_checked_on_the_device(svo, golden, nq):
         with pytest.raises(svo.SvoError) as e:
             svo.VoxelOctree.build_from_mesh(a, False, c, i, 64, threads=8)
         assert e.value.code == code
+
+
+@pytest.mark.parametrize("depth", [40, 41])
+@pytest.mark.parametrize("black", [0.0, 0.5, 1.0])
+def test_mesh_voxels_with_an_empty_word(svo, golden, black, depth):
+    """Voxels whose material packs to the empty word are no leaves: none, some
+    or all of a mesh's, in volumes whose last slice is scanned (an even depth)
+    and is not (an odd one), against the oracle's build."""
+    rng = np.random.default_rng(23)
+    n, res = 1500, 64
+    v = (rng.uniform(0.1, 0.9, (n, 1, 3)) + rng.normal(scale=0.02, size=(n, 3, 3))).astype(np.float32)
+    v[:2] = [[[0, 0, 0], [0.02, 0, 0], [0, 0.02, 0]], [[1, 1, 1], [0.98, 1, 1], [1, 0.98, 1]]]
+    v = np.clip(v, 0, 1)
+    v[..., 2] *= (depth - 2 + 0.5) / (res - 2)
+    tab = np.zeros((n, 3, 9), np.float32)
+    tab[..., :3], tab[..., 3:6], tab[..., 6:] = v, (1, 0, 0), 200.0
+    dark = rng.random(n) < black
+    tab[dark, :, 3:6], tab[dark, :, 6:] = (1, -1, -1), 0.0
+    tab = tab.reshape(-1, 9)
+    counts, idx = np.full(n, 3, np.int32), np.arange(3 * n, dtype=np.int32)
+    print(f"[gpu] mesh with {int(dark.sum())} of {n} triangles black, depth {depth}", flush=True)
+    t = svo.VoxelOctree.build_from_mesh(tab, True, counts, idx, res, threads=8, memory_budget=1 << 30)
+    center, words, _ = orc.Mesh(tab, True, counts, idx).build(res, 8, 1 << 30)
+    assert np.array_equal(t.words(), words) and np.array_equal(t.center(), center)
+    assert (t.build_stats()["leaves"] == 0) == (black == 1.0)
+    assert t.center()[2] == np.float32(depth) * np.float32(0.5) / np.float32(64)
