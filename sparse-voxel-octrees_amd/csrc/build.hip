@@ -870,18 +870,24 @@ __device__ __forceinline__ void fold_voxel(const uint64_t *__restrict__ keys, ui
 // Voxels per wave in fold_kernel: a lane that has folded its voxel takes the
 // chunk's next one, so a wave's lanes stay busy while their voxels' triangle
 // counts differ (one lane per voxel would run every lane as long as the
-// voxel with the most triangles).
-constexpr int kFoldChunk = 512;
-constexpr uint64_t kFoldVoxelsPerBlock = uint64_t(kFoldChunk) * (kThreads / 64);
+// voxel with the most triangles). Volumes too small for kFoldWaves waves of 512
+// voxels (8 per SIMD) take fewer per wave, down to one per lane: at 512 a
+// 256^3 mesh's 0.1 M voxels gave 4 in 5 SIMDs no wave, and each wave 8 or more
+// rounds of dependent loads: 72 us of a 1,107 us build, now 1,061; a 64^3 one
+// 818 -> 776; 2048^3 has 18 K waves either way (0.87 ms, bound by its VALU work).
+constexpr uint64_t kFoldChunk = 512, kFoldWaves = 8192;
+inline uint64_t fold_chunk(uint64_t S) {
+    return std::min(kFoldChunk, std::max<uint64_t>(64, (S / kFoldWaves + 63) / 64 * 64));
+}
 
 __global__ void __launch_bounds__(kThreads) fold_kernel(const uint64_t *__restrict__ keys, const uint64_t *__restrict__ segStart, uint64_t S,
-                            int tribits, const float *__restrict__ pos, const float *__restrict__ nrm,
+                            uint64_t chunk, int tribits, const float *__restrict__ pos, const float *__restrict__ nrm,
                             const float *__restrict__ col, MeshParams mp, uint64_t *__restrict__ vkey,
                             uint32_t *__restrict__ vword, uint8_t *__restrict__ vcount) {
     const int lane = threadIdx.x & 63;
-    const uint64_t base = (uint64_t(blockIdx.x) * (kThreads / 64) + (threadIdx.x >> 6)) * kFoldChunk;
+    const uint64_t base = (uint64_t(blockIdx.x) * (kThreads / 64) + (threadIdx.x >> 6)) * chunk;
     if (base >= S) return;
-    const uint64_t end = min(base + uint64_t(kFoldChunk), S);
+    const uint64_t end = min(base + chunk, S);
     const uint64_t triMask = (uint64_t(1) << tribits) - 1;
     uint64_t next = base;  // the chunk's next unassigned voxel (wave-uniform)
     uint64_t v = 0, k = 0, e = 0;
@@ -2522,10 +2528,11 @@ static int mesh_core(Arena &ar, float *dv, int64_t nverts, int has_normals, int3
     hipLaunchKernelGGL(set_u64_kernel, dim3(1), dim3(1), 0, st, segStart + V, K);
     if (sink) return write_volume(ar, g, mp, tribits, keys2, segStart, V, pos, nrm, col, sliceZ, sink->fp);
     if ((r = ar.alloc(vkey, V)) || (r = ar.alloc(vword, V)) || (r = ar.alloc(vcount, V))) return r;
-    if (V)
-        hipLaunchKernelGGL(fold_kernel, dim3(unsigned((V + kFoldVoxelsPerBlock - 1) / kFoldVoxelsPerBlock)), dim3(kThreads),
-                           0, st, keys2, segStart, V, tribits, pos, nrm,
-                           col, mp, vkey, vword, vcount);
+    if (V) {
+        const uint64_t chunk = fold_chunk(V), perBlock = chunk * (kThreads / 64);
+        hipLaunchKernelGGL(fold_kernel, dim3(unsigned((V + perBlock - 1) / perBlock)), dim3(kThreads), 0, st, keys2, segStart,
+                           V, chunk, tribits, pos, nrm, col, mp, vkey, vword, vcount);
+    }
     HIP_TRY(hipGetLastError());
 
     uint64_t *lkey, L;
