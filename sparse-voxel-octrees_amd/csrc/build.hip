@@ -1090,95 +1090,107 @@ __global__ void dense_children_kernel(const uint64_t *__restrict__ child, const 
 // children occupies n*(1+large) words for its child block plus its children's
 // subtrees S. Child i's offset from its own slot, before the node's far words,
 // is n - i + sum_{j<i} S(c_j); the node needs far pointers (large) if any
-// exceeds 0x3FFF, and then every child slot takes a second word.
-__global__ void size_kernel(const uint32_t *__restrict__ mask, const uint64_t *__restrict__ start,
-                            const uint64_t *__restrict__ nptr, int leafParents, const uint64_t *__restrict__ childS,
-                            uint64_t *__restrict__ S, uint8_t *__restrict__ large) {
+// exceeds 0x3FFF, and then every child slot takes a second word. Taken over a
+// node's children in order; childless and leaf-parent nodes are never large.
+struct SubtreeSum {
+    uint64_t words = 0;  // of the children's subtrees so far
+    int64_t most = 0;    // largest of (words before child i) - i
+    __device__ void add(uint32_t i, uint64_t childS) {
+        most = max(most, int64_t(words) - int64_t(i));
+        words += childS;
+    }
+    __device__ bool large(uint32_t n) const { return words && int64_t(n) + most > 0x3FFF; }
+    __device__ uint64_t size(uint32_t n) const { return uint64_t(n) * (large(n) ? 2 : 1) + words; }
+};
+
+// A level's child masks carry the large flag above the eight child bits.
+constexpr uint32_t kLargeBit = 0x100u;
+
+// Sizes of a level whose masks are complete only after its pass (the dense
+// one); the others take theirs with their parents (parent_emit_kernel).
+__global__ void size_kernel(uint32_t *__restrict__ mask, const uint64_t *__restrict__ start,
+                            const uint64_t *__restrict__ nptr, const uint64_t *__restrict__ childS,
+                            uint64_t *__restrict__ S) {
     uint64_t k = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (k >= *nptr) return;
-    const uint32_t c = __popc(mask[k]);
-    if (leafParents || c == 0) {
-        S[k] = c;
-        large[k] = 0;
-        return;
-    }
-    uint64_t acc = 0, maxOff = 0;
-    const uint64_t s0 = start[k];
-    for (uint32_t i = 0; i < c; ++i) {
-        const uint64_t off = uint64_t(c - i) + acc;
-        if (off > maxOff) maxOff = off;
-        acc += childS[s0 + i];
-    }
-    const bool lg = maxOff > 0x3FFF;
-    large[k] = lg ? 1 : 0;
-    S[k] = uint64_t(c) * (lg ? 2 : 1) + acc;
+    const uint32_t m = mask[k], c = __popc(m);
+    SubtreeSum sum;
+    if (childS)
+        for (uint32_t i = 0; i < c; ++i) sum.add(i, childS[start[k] + i]);
+    if (sum.large(c)) mask[k] = m | kLargeBit;
+    S[k] = sum.size(c);
 }
 
-// Placement, top-down: a node at `pos` whose child block starts at `B` puts
-// child i at B + i*(1+large); that child's own block starts after the node's
-// whole child block and the subtrees of children 0..i-1.
-__global__ void place_kernel(const uint32_t *__restrict__ mask, const uint64_t *__restrict__ start,
-                             const uint64_t *__restrict__ nptr, const uint64_t *__restrict__ B,
-                             const uint8_t *__restrict__ large, const uint64_t *__restrict__ childS, int childLeaves,
-                             uint64_t *__restrict__ childPos, uint64_t *__restrict__ childB,
-                             uint8_t *__restrict__ childFar) {
-    uint64_t k = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (k >= *nptr) return;
-    const uint32_t c = __popc(mask[k]);
-    if (c == 0) return;
-    const uint64_t per = large[k] ? 2 : 1;
-    const uint64_t b = B[k], s0 = start[k];
-    uint64_t acc = 0;
-    for (uint32_t i = 0; i < c; ++i) {
-        childPos[s0 + i] = b + i * per;
-        if (!childLeaves) {
-            childB[s0 + i] = b + uint64_t(c) * per + acc;
-            childFar[s0 + i] = large[k];
-            acc += childS[s0 + i];
-        }
-    }
-}
+// A level's arrays on the device. pos: word index of the node, the top bit set
+// where its slot carries a far word; B: word index of its child block.
+struct LevelArrays {
+    uint64_t *cnt, *key, *start, *S, *pos, *B;
+    uint32_t *mask;
+};
+constexpr uint64_t kFarSlot = uint64_t(1) << 63;
 
-// Descriptor word (and far word) of every node of one level.
+// Placement and output of one node: its descriptor (and far word), then its
+// children: a leaf parent's words are written at once, other children get
+// their slot B + i*(1+large) and their own block, which starts after the
+// node's whole child block and the subtrees of children 0..i-1.
 // Positions are checked against the word count W; a violation (which the
 // size/placement arithmetic excludes) is reported instead of written.
-__global__ void write_nodes_kernel(const uint32_t *__restrict__ mask, const uint64_t *__restrict__ nptr,
-                                   const uint64_t *__restrict__ pos, const uint64_t *__restrict__ B,
-                                   const uint8_t *__restrict__ large, const uint8_t *__restrict__ far, int leafParents,
-                                   uint32_t *__restrict__ out, uint64_t W, uint32_t *__restrict__ bad) {
-    uint64_t k = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (k >= *nptr) return;
-    const uint32_t m = mask[k];
-    uint32_t w = (m << 8) | (leafParents ? 0u : m);
-    if (large[k]) w |= 0x10000u;
-    const uint64_t p = pos[k];
-    const uint64_t off = B[k] - p;
+__device__ __forceinline__ void write_node(uint64_t k, const LevelArrays &a, const uint32_t *leafWord,
+                                           const uint64_t *childS, uint64_t *childPos, uint64_t *childB, uint32_t *out,
+                                           uint64_t W, uint32_t *bad) {
+    const uint32_t m = a.mask[k] & 0xFFu, n = __popc(m);
+    const bool large = (a.mask[k] & kLargeBit) != 0, far = (a.pos[k] & kFarSlot) != 0;
+    const uint64_t p = a.pos[k] & ~kFarSlot, b = a.B[k], s0 = a.start[k];
     // the traversal reads child slot B + (non-leaf children before it) * (1 + large)
     // or B + (children before it) for a leaf: the block must follow the node
     // and end inside the array
-    const uint64_t kids = uint64_t(__popc(m)), extent = leafParents ? kids : kids * (large[k] ? 2u : 1u);
-    if (p >= W || (far[k] && p + 1 >= W) || (kids && (B[k] <= p || B[k] > W || extent > W - B[k]))) {
+    const uint64_t per = large ? 2 : 1, extent = uint64_t(n) * per;
+    if (p >= W || (far && p + 1 >= W) || (n && (b <= p || b > W || extent > W - b))) {
         atomicOr(bad, 1u);
         return;
     }
-    if (far[k]) {
+    const uint64_t off = b - p;
+    uint32_t w = (m << 8) | (leafWord ? 0u : m);
+    if (large) w |= 0x10000u;
+    if (far) {
         w |= 0x20000u | uint32_t((off >> 32) << 18);
         out[p + 1] = uint32_t(off);
     } else {
         w |= uint32_t(off << 18);
     }
     out[p] = w;
-}
-
-__global__ void write_leaves_kernel(const uint32_t *__restrict__ word, uint64_t n, const uint64_t *__restrict__ pos,
-                                    uint32_t *__restrict__ out, uint64_t W, uint32_t *__restrict__ bad) {
-    uint64_t k = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    if (pos[k] >= W) {
-        atomicOr(bad, 1u);
+    // every load before the first store, which may alias it for all the
+    // compiler knows
+    if (leafWord) {
+        uint32_t v[8];
+#pragma unroll
+        for (uint32_t i = 0; i < 8; ++i) v[i] = i < n ? leafWord[s0 + i] : 0;
+#pragma unroll
+        for (uint32_t i = 0; i < 8; ++i)
+            if (i < n) out[b + i] = v[i];
         return;
     }
-    out[pos[k]] = word[k];
+    uint64_t v[8];
+#pragma unroll
+    for (uint32_t i = 0; i < 8; ++i) v[i] = i < n ? childS[s0 + i] : 0;
+    uint64_t at = b + extent;
+#pragma unroll
+    for (uint32_t i = 0; i < 8; ++i)
+        if (i < n) {
+            childPos[s0 + i] = (b + i * per) | (large ? kFarSlot : 0);
+            childB[s0 + i] = at;
+            at += v[i];
+        }
+}
+
+// One level, a thread per node. One pass writes the level and places its
+// children: as passes of their own over the nodes, their children's slots and
+// the leaves, a 2048^3 mesh took 370 us and 24 launches, this 200 and 11.
+__global__ void __launch_bounds__(kThreads) write_level_kernel(LevelArrays a, uint64_t n, LevelArrays child,
+                                                               const uint32_t *leafWord, uint32_t *out, uint64_t W,
+                                                               uint32_t *bad) {
+    const uint64_t k = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (k < n) write_node(k, a, leafWord, child.S, child.pos, child.B, out, W, bad);
 }
 
 __global__ void fill_u32_kernel(uint32_t *p, uint64_t n, uint32_t v) {
@@ -1186,24 +1198,19 @@ __global__ void fill_u32_kernel(uint32_t *p, uint64_t n, uint32_t v) {
     if (i < n) p[i] = v;
 }
 
-// The root level of an empty tree or the root's placement: one node.
-__global__ void root_init_kernel(uint64_t *key, uint64_t *start, uint32_t *mask, uint64_t *cnt) {
-    *key = 0;
-    *start = 0;
-    *mask = 0;
-    *cnt = 1;
+// The root of an empty tree, a node of its own.
+__global__ void root_init_kernel(LevelArrays root) {
+    *root.key = 0;
+    *root.start = 0;
+    *root.mask = 0;
+    *root.S = 0;
+    *root.cnt = 1;
 }
 
-__global__ void root_place_kernel(uint64_t *pos, uint64_t *B, uint8_t *far) {
+__global__ void root_place_kernel(uint64_t *pos, uint64_t *B, uint32_t *bad) {
     *pos = 0;
     *B = 1;
-    *far = 0;
-}
-
-// {root subtree size, root level count} for the host, in one read.
-__global__ void root_report_kernel(const uint64_t *S0, const uint64_t *cnt0, uint64_t *out) {
-    out[0] = *S0;
-    out[1] = *cnt0;
+    *bad = 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -1559,89 +1566,137 @@ __global__ void __launch_bounds__(kThreads) scan_down_kernel(const In *__restric
 // i == 0 or its key differs from key i - 1. A compaction in the scan's three
 // passes with the head flags computed from the keys in the first and third
 // (no flag or index arrays): the first counts each tile's heads, the second
-// scans the tile counts, the third gives each head its index j among the
-// heads and calls emit(j, i, n).
-__device__ __forceinline__ uint32_t run_head_flags(const uint64_t *__restrict__ keys, uint64_t first, uint64_t n,
-                                                   int shift) {
-    uint64_t k[kScanItems];
-    if (first + kScanItems <= n) {
+// scans the tile counts, the third lists its tile's heads in LDS and takes
+// them a thread each, so that loads, stores and the work per head stay dense
+// (with eight neighbouring keys per thread, the threads' loads lay 64 bytes
+// apart and each thread went through its own heads: a 2048^3 mesh's segment
+// starts, 24 M keys, took 106 us where this takes 81, its two largest levels'
+// parents 128 + 45 and their sizes, in passes of their own, 15 + 19, where this
+// takes 55 + 37 for both). Bound by memory on the large levels, by its launches
+// on the small ones.
+//
+// Head flags of the tile at `base`: bits[k] for the wave's keys base +
+// k * kThreads + thread; the keys themselves go to `tile` where it is given.
+__device__ __forceinline__ void tile_flags(const uint64_t *__restrict__ keys, uint64_t base, uint64_t n, int shift,
+                                           uint64_t bits[kScanItems], uint64_t *tile) {
+    uint64_t key[kScanItems], prev[kScanItems];
 #pragma unroll
-        for (int q = 0; q < kScanItems; q += 2) {
-            const ulonglong2 v = *reinterpret_cast<const ulonglong2 *>(keys + first + q);
-            k[q] = v.x;
-            k[q + 1] = v.y;
-        }
-    } else {
-#pragma unroll
-        for (int q = 0; q < kScanItems; ++q) k[q] = first + q < n ? keys[first + q] : 0;
+    for (int k = 0; k < kScanItems; ++k) {
+        const uint64_t i = base + uint64_t(k) * kThreads + threadIdx.x;
+        key[k] = i < n ? keys[i] : 0;
+        prev[k] = (threadIdx.x & 63) == 0 && i && i < n ? keys[i - 1] : 0;
     }
-    uint64_t prev = (first && first <= n) ? keys[first - 1] >> shift : 0;
-    uint32_t flags = 0;
 #pragma unroll
-    for (int q = 0; q < kScanItems; ++q) {
-        const uint64_t cur = k[q] >> shift;
-        if (first + q < n && (first + q == 0 || cur != prev)) flags |= 1u << q;
-        prev = cur;
+    for (int k = 0; k < kScanItems; ++k) {
+        const uint64_t i = base + uint64_t(k) * kThreads + threadIdx.x;
+        const uint64_t left = __shfl_up(key[k], 1), before = (threadIdx.x & 63) ? left : prev[k];
+        bits[k] = __ballot(i < n && (i == 0 || (key[k] >> shift) != (before >> shift)));
+        if (tile) tile[k * kThreads + int(threadIdx.x)] = key[k];
     }
-    return flags;
+}
+
+// The tile's heads, by position in the tile, into head[]; returns their count.
+// at: kScanItems * kThreads / 64 words.
+__device__ __forceinline__ uint32_t tile_heads(const uint64_t bits[kScanItems], uint16_t *head, uint32_t *at) {
+    constexpr int kWaves = kThreads / 64, kGroups = kScanItems * kWaves;
+    static_assert(kGroups <= 64, "one wave scans the groups");
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (lane == 0)
+#pragma unroll
+        for (int k = 0; k < kScanItems; ++k) at[k * kWaves + wave] = uint32_t(__popcll(bits[k]));
+    __syncthreads();
+    uint32_t total = 0, first[kScanItems];
+#pragma unroll
+    for (int g = 0; g < kGroups; ++g) {
+        if (g % kWaves == wave) first[g / kWaves] = total;
+        total += at[g];
+    }
+    const uint64_t below = (uint64_t(1) << lane) - 1;
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k)
+        if (bits[k] >> lane & 1) head[first[k] + uint32_t(__popcll(bits[k] & below))] = uint16_t(k * kThreads + threadIdx.x);
+    __syncthreads();
+    return total;
 }
 
 __global__ void __launch_bounds__(kThreads) run_sums_kernel(const uint64_t *__restrict__ keys,
                                                             const uint64_t *__restrict__ nptr, int shift,
                                                             uint64_t *__restrict__ sums) {
-    __shared__ uint64_t lds[kThreads / 64];
+    __shared__ uint32_t part[kThreads / 64];
     const uint64_t n = *nptr;
     const uint64_t base = uint64_t(blockIdx.x) * kScanTile;
     if (base >= n) {
         if (threadIdx.x == 0) sums[blockIdx.x] = 0;
         return;
     }
-    const uint32_t flags = run_head_flags(keys, base + uint64_t(threadIdx.x) * kScanItems, n, shift);
-    uint64_t total;
-    block_exclusive(uint64_t(__builtin_popcount(flags)), lds, &total);
-    if (threadIdx.x == 0) sums[blockIdx.x] = total;
-}
-
-template <typename Emit>
-__global__ void __launch_bounds__(kThreads) run_emit_kernel(const uint64_t *__restrict__ keys,
-                                                            const uint64_t *__restrict__ nptr, int shift,
-                                                            const uint64_t *__restrict__ offs, Emit emit) {
-    __shared__ uint64_t lds[kThreads / 64];
-    const uint64_t n = *nptr;
-    const uint64_t base = uint64_t(blockIdx.x) * kScanTile;
-    if (base >= n) return;
-    const uint64_t first = base + uint64_t(threadIdx.x) * kScanItems;
-    uint32_t flags = run_head_flags(keys, first, n, shift);
-    uint64_t total;
-    uint64_t j = offs[blockIdx.x] + block_exclusive(uint64_t(__builtin_popcount(flags)), lds, &total);
-    for (; flags; flags &= flags - 1, ++j) emit(j, first + uint64_t(__builtin_ctz(flags)), n);
+    uint64_t bits[kScanItems];
+    tile_flags(keys, base, n, shift, bits, nullptr);
+    uint32_t count = 0;
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) count += uint32_t(__popcll(bits[k]));
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = count;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint64_t total = 0;
+        for (int w = 0; w < kThreads / 64; ++w) total += part[w];
+        sums[blockIdx.x] = total;
+    }
 }
 
 // The fold's segments: segStart[j] = the first candidate of voxel j.
-struct SegmentEmit {
-    uint64_t *segStart;
-    __device__ void operator()(uint64_t j, uint64_t i, uint64_t) const { segStart[j] = i; }
-};
+__global__ void __launch_bounds__(kThreads) segment_emit_kernel(const uint64_t *__restrict__ keys,
+                                                                const uint64_t *__restrict__ nptr, int shift,
+                                                                const uint64_t *__restrict__ offs,
+                                                                uint64_t *__restrict__ segStart) {
+    __shared__ uint16_t head[kScanTile];
+    __shared__ uint32_t at[kScanItems * kThreads / 64];
+    const uint64_t n = *nptr;
+    const uint64_t base = uint64_t(blockIdx.x) * kScanTile;
+    if (base >= n) return;
+    uint64_t bits[kScanItems];
+    tile_flags(keys, base, n, shift, bits, nullptr);
+    const uint32_t heads = tile_heads(bits, head, at);
+    const uint64_t j = offs[blockIdx.x];
+    for (uint32_t h = threadIdx.x; h < heads; h += kThreads) segStart[j + h] = base + head[h];
+}
 
-// A level's parents from the sorted child keys: parent j's key, first child
-// and child mask (its children, at most 8 since keys are unique, follow i).
-struct ParentEmit {
-    const uint64_t *child;
-    uint64_t *pkey, *pstart;
-    uint32_t *pmask;
-    __device__ void operator()(uint64_t j, uint64_t i, uint64_t n) const {
-        const uint64_t parent = child[i] >> 3;
-        uint32_t mask = 1u << uint32_t(child[i] & 7);
-        for (uint64_t q = i + 1; q < n && q < i + 8; ++q) {
-            const uint64_t k = child[q];
+// A level's parents from the sorted child keys: parent j's key, first child,
+// child mask and subtree size (its children, at most 8 since keys are unique,
+// follow the head). Leaves have no sizes.
+template <bool Leaves>
+__global__ void __launch_bounds__(kThreads) parent_emit_kernel(LevelArrays child, LevelArrays p,
+                                                               const uint64_t *__restrict__ offs) {
+    __shared__ uint64_t key[kScanTile + 8], size[Leaves ? 1 : kScanTile + 8];
+    __shared__ uint16_t head[kScanTile];
+    __shared__ uint32_t at[kScanItems * kThreads / 64];
+    const uint64_t n = *child.cnt;
+    const uint64_t base = uint64_t(blockIdx.x) * kScanTile;
+    if (base >= n) return;
+    uint64_t bits[kScanItems];
+    tile_flags(child.key, base, n, 3, bits, key);
+    for (uint64_t t = threadIdx.x; t < 8; t += kThreads)
+        if (base + kScanTile + t < n) key[kScanTile + t] = child.key[base + kScanTile + t];
+    if constexpr (!Leaves)
+        for (uint64_t t = threadIdx.x; t < kScanTile + 8; t += kThreads) size[t] = base + t < n ? child.S[base + t] : 0;
+    const uint32_t heads = tile_heads(bits, head, at);
+    const uint64_t j = offs[blockIdx.x];
+    for (uint32_t h = threadIdx.x; h < heads; h += kThreads) {
+        const uint32_t i = head[h];
+        const uint64_t parent = key[i] >> 3;
+        uint32_t mask = 0, c = 0;
+        SubtreeSum sum;
+        for (; c < 8 && base + i + c < n; ++c) {
+            const uint64_t k = key[i + c];
             if ((k >> 3) != parent) break;
             mask |= 1u << uint32_t(k & 7);
+            if constexpr (!Leaves) sum.add(c, size[i + c]);
         }
-        pkey[j] = parent;
-        pstart[j] = i;
-        pmask[j] = mask;
+        p.key[j + h] = parent;
+        p.start[j + h] = base + i;
+        p.mask[j + h] = mask | (sum.large(c) ? kLargeBit : 0);
+        p.S[j + h] = sum.size(c);
     }
-};
+}
 
 __global__ void set_u64_kernel(uint64_t *p, uint64_t v) { *p = v; }
 
@@ -1688,22 +1743,20 @@ int exclusive_scan_dev(Arena &ar, const In *in, uint64_t *out, const uint64_t *n
     return SVO_OK;
 }
 
-// Run heads of keys[0, *nptr) (sorted; runs of equal keys >> shift): emit(j,
-// i, n) for each head i, j its index among the heads; *total (device) = the
-// head count. `bound` (host) bounds *nptr and sizes the grids.
+// Run heads of keys[0, *nptr) (sorted; runs of equal keys >> shift): each
+// tile's heads before it in sums[], which emit(blocks, sums) reads; *total
+// (device) = the head count. `bound` (host) bounds *nptr and sizes the grids.
 template <typename Emit>
 int run_heads(Arena &ar, const uint64_t *keys, const uint64_t *nptr, uint64_t bound, int shift, uint64_t *total,
               const Emit &emit, hipStream_t s) {
     const uint64_t nb = std::max<uint64_t>(1, (bound + kScanTile - 1) / kScanTile);
     if (nb > 0x7FFFFFFFull) return fail(SVO_ERR_LIMIT, "builder: scan too large");
-    if (reinterpret_cast<uintptr_t>(keys) % 16)
-        return fail(SVO_ERR_DEVICE, "builder: key arrays must be 16-byte aligned (internal error)");
     uint64_t *sums;
     int r = ar.alloc(sums, nb);
     if (r) return r;
     hipLaunchKernelGGL(run_sums_kernel, dim3(unsigned(nb)), dim3(kThreads), 0, s, keys, nptr, shift, sums);
     hipLaunchKernelGGL(scan_block_sums_kernel, dim3(1), dim3(kSumThreads), 0, s, sums, nb, total);
-    hipLaunchKernelGGL(run_emit_kernel<Emit>, dim3(unsigned(nb)), dim3(kThreads), 0, s, keys, nptr, shift, sums, emit);
+    emit(unsigned(nb), sums);
     HIP_TRY(hipGetLastError());
     ar.release(sums);
     return SVO_OK;
@@ -1748,19 +1801,9 @@ int fill32(uint32_t *p, uint64_t n, uint32_t v, hipStream_t s) {
     return SVO_OK;
 }
 
-struct Level {
-    uint64_t n = 0;             // node count when known on the host (the leaves)
-    uint64_t bound = 0;         // host upper bound of the node count (sizes arrays and grids)
-    uint64_t *cnt = nullptr;    // node count, device word
-    uint64_t *key = nullptr;
-    uint32_t *mask = nullptr;   // child mask (nodes above the leaves)
-    uint64_t *start = nullptr;  // index of the first child in the level below
-    uint64_t *S = nullptr;      // subtree size (words after the node's slot)
-    uint8_t *large = nullptr;
-    uint64_t *pos = nullptr;    // word index of the node
-    uint64_t *B = nullptr;      // word index of the node's child block
-    uint8_t *far = nullptr;     // the node's slot carries a far word
-    uint32_t *word = nullptr;   // leaves: material word
+struct Level : LevelArrays {  // the leaves' S, pos and B stay null
+    uint64_t bound = 0;  // node count, a host upper bound of it until it is read (sizes arrays and grids)
+    Level() : LevelArrays{} {}
 };
 
 // Large copies between pageable host memory and the device go through pinned
@@ -1879,21 +1922,27 @@ int emit_tree(Arena &ar, const Geometry &g, uint64_t *leafKey, uint32_t *leafWor
               const uint32_t *blockFlags, hipStream_t st, svo_octree &out) {
     const int D = g.depth;
     std::vector<Level> lv(size_t(D) + 1);
-    lv[D].n = L;
     lv[D].bound = L;
     lv[D].key = leafKey;
-    lv[D].word = leafWord;
     const int cacheLevel = D - g.cacheLog;  // nodes of edge `cache`
     const bool multi = g.cacheLog < D;
     int r;
-    uint64_t *cnts;  // every level's node count, one word each, read together once the levels exist
-    if ((r = ar.alloc(cnts, uint64_t(D) + 1))) return r;
+    uint64_t *cnts;  // every level's node count, one word each, then the root's size: read together
+    if ((r = ar.alloc(cnts, uint64_t(D) + 2))) return r;
     for (int d = 0; d <= D; ++d) lv[size_t(d)].cnt = cnts + d;
     hipLaunchKernelGGL(set_u64_kernel, dim3(1), dim3(1), 0, st, lv[D].cnt, L);
+    auto level_arrays = [&](Level &p, bool root) {
+        int q;
+        if (root) p.S = cnts + D + 1;
+        else if ((q = ar.alloc(p.S, p.bound))) return q;
+        if ((q = ar.alloc(p.key, p.bound)) || (q = ar.alloc(p.start, p.bound))) return q;
+        return ar.alloc(p.mask, p.bound);
+    };
     // Levels bottom-up. Node counts stay on the device: each level's arrays
     // are sized by a host bound (no more nodes than the level below, nor than
-    // 8^d cells), so no level waits for the host. `empty`: the level below is
-    // known on the host to hold no node (a tree without leaves).
+    // 8^d cells), so no level waits for the host; its keys are given back once
+    // the level above has them. `empty`: the level below is known on the host
+    // to hold no node (a tree without leaves).
     bool empty = L == 0;
     for (int d = D - 1; d >= 0; --d) {
         Level &c = lv[d + 1];
@@ -1908,14 +1957,17 @@ int emit_tree(Arena &ar, const Geometry &g, uint64_t *leafKey, uint32_t *leafWor
                 hipLaunchKernelGGL(dense_mark_kernel, dim3(grid_for(c.bound)), dim3(kThreads), 0, st, c.key, c.cnt, dense);
             if ((r = exclusive_scan(ar, dense, at, cells, st, p.cnt))) return r;
             p.bound = cells;
-            if ((r = ar.alloc(p.key, p.bound)) || (r = ar.alloc(p.start, p.bound)) || (r = ar.alloc(p.mask, p.bound)))
-                return r;
+            if ((r = level_arrays(p, d == 0))) return r;
             if ((r = fill32(p.mask, p.bound, 0, st))) return r;
             hipLaunchKernelGGL(dense_compact_kernel, dim3(grid_for(cells)), dim3(kThreads), 0, st, dense, cells, at,
                                p.key, slot);
             if (c.bound)
                 hipLaunchKernelGGL(dense_children_kernel, dim3(grid_for(c.bound)), dim3(kThreads), 0, st, c.key, c.cnt,
                                    slot, p.start, p.mask);
+            hipLaunchKernelGGL(size_kernel, dim3(grid_for(cells)), dim3(kThreads), 0, st, p.mask, p.start, p.cnt, c.S, p.S);
+            ar.release(dense);
+            ar.release(at);
+            ar.release(slot);
             if (L == 0) {
                 // no leaves: the table level alone decides whether nodes exist
                 uint64_t nTable = 0;
@@ -1926,47 +1978,34 @@ int emit_tree(Arena &ar, const Geometry &g, uint64_t *leafKey, uint32_t *leafWor
             // an empty level below: only the root remains (an empty tree)
             if (empty) {
                 p.bound = d == 0 ? 1 : 0;
-                if ((r = ar.alloc(p.key, 1)) || (r = ar.alloc(p.start, 1)) || (r = ar.alloc(p.mask, 1))) return r;
-                if (d == 0) hipLaunchKernelGGL(root_init_kernel, dim3(1), dim3(1), 0, st, p.key, p.start, p.mask, p.cnt);
+                if ((r = level_arrays(p, d == 0))) return r;
+                if (d == 0) hipLaunchKernelGGL(root_init_kernel, dim3(1), dim3(1), 0, st, LevelArrays(p));
                 else hipLaunchKernelGGL(set_u64_kernel, dim3(1), dim3(1), 0, st, p.cnt, uint64_t(0));
                 continue;
             }
             p.bound = d < 21 ? std::min(c.bound, uint64_t(1) << (3 * d)) : c.bound;
-            if ((r = ar.alloc(p.key, p.bound)) || (r = ar.alloc(p.start, p.bound)) || (r = ar.alloc(p.mask, p.bound)))
-                return r;
+            if ((r = level_arrays(p, d == 0))) return r;
             // every parent below the count is written once (by its first child)
-            if ((r = run_heads(ar, c.key, c.cnt, c.bound, 3, p.cnt, ParentEmit{c.key, p.key, p.start, p.mask}, st)))
-                return r;
+            auto parents = [&](unsigned blocks, const uint64_t *sums) {
+                auto kernel = d == D - 1 ? parent_emit_kernel<true> : parent_emit_kernel<false>;
+                hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), 0, st, LevelArrays(c), LevelArrays(p), sums);
+            };
+            if ((r = run_heads(ar, c.key, c.cnt, c.bound, 3, p.cnt, parents, st))) return r;
         }
+        ar.release(c.key);
         HIP_TRY(hipGetLastError());
     }
 
-    // the level counts (one read): the size, placement and scatter arrays
-    // below are allocated and launched at the exact counts
-    {
-        std::vector<uint64_t> n(size_t(D) + 1);
-        if ((r = read_words(cnts, n.data(), D + 1, st))) return r;
-        for (int d = 0; d < D; ++d) {
-            if (n[size_t(d)] > lv[size_t(d)].bound) return fail(SVO_ERR_DEVICE, "builder: level above its bound (internal error)");
-            lv[size_t(d)].bound = n[size_t(d)];
-        }
+    // the level counts and the root's size, in the one round trip of the level
+    // passes: the arrays below are allocated and launched at the exact counts
+    std::vector<uint64_t> report(size_t(D) + 2);
+    if ((r = read_words(cnts, report.data(), D + 2, st))) return r;
+    for (int d = 0; d < D; ++d) {
+        if (report[size_t(d)] > lv[size_t(d)].bound) return fail(SVO_ERR_DEVICE, "builder: level above its bound (internal error)");
+        lv[size_t(d)].bound = report[size_t(d)];
     }
-    // sizes, bottom-up
-    for (int d = D - 1; d >= 0; --d) {
-        Level &p = lv[d];
-        if ((r = ar.alloc(p.S, p.bound)) || (r = ar.alloc(p.large, p.bound))) return r;
-        if (p.bound)
-            hipLaunchKernelGGL(size_kernel, dim3(grid_for(p.bound)), dim3(kThreads), 0, st, p.mask, p.start, p.cnt,
-                               int(d == D - 1), lv[d + 1].S, p.S, p.large);
-        HIP_TRY(hipGetLastError());
-    }
-    // the one round trip of the level passes: the word count sizes the array
-    uint64_t *rep, report[2] = {0, 0};
-    if ((r = ar.alloc(rep, 2))) return r;
-    hipLaunchKernelGGL(root_report_kernel, dim3(1), dim3(1), 0, st, lv[0].S, lv[0].cnt, rep);
-    if ((r = read_words(rep, report, 2, st))) return r;
-    if (report[1] != 1) return fail(SVO_ERR_DEVICE, "builder: root level does not hold one node");
-    const uint64_t W = 1 + report[0];
+    if (report[0] != 1) return fail(SVO_ERR_DEVICE, "builder: root level does not hold one node");
+    const uint64_t W = 1 + report[size_t(D) + 1];
     // the word array, allocated before the host array below: both map memory
     // into the process, and a device allocation waits while other threads
     // populate host pages
@@ -1995,35 +2034,19 @@ int emit_tree(Arena &ar, const Geometry &g, uint64_t *leafKey, uint32_t *leafWor
         }
     });
 
-    // placement, top-down
-    {
-        Level &root = lv[0];
-        if ((r = ar.alloc(root.pos, 1)) || (r = ar.alloc(root.B, 1)) || (r = ar.alloc(root.far, 1))) return r;
-        hipLaunchKernelGGL(root_place_kernel, dim3(1), dim3(1), 0, st, root.pos, root.B, root.far);
-    }
-    for (int d = 0; d < D; ++d) {
-        Level &p = lv[d], &c = lv[d + 1];
-        const bool childLeaves = d + 1 == D;
-        if ((r = ar.alloc(c.pos, c.bound))) return r;
-        if (!childLeaves && ((r = ar.alloc(c.B, c.bound)) || (r = ar.alloc(c.far, c.bound)))) return r;
-        if (p.bound)
-            hipLaunchKernelGGL(place_kernel, dim3(grid_for(p.bound)), dim3(kThreads), 0, st, p.mask, p.start, p.cnt,
-                               p.B, p.large, childLeaves ? nullptr : c.S, int(childLeaves), c.pos, c.B, c.far);
-        HIP_TRY(hipGetLastError());
-    }
-
-    // scatter
+    // placement and output, top-down
     uint32_t *bad;
-    if ((r = ar.alloc(bad, 1)) || (r = fill32(bad, 1, 0, st))) return r;
+    if ((r = ar.alloc(bad, 1))) return r;
+    for (int d = 0; d < D; ++d)
+        if ((r = ar.alloc(lv[size_t(d)].pos, lv[size_t(d)].bound)) || (r = ar.alloc(lv[size_t(d)].B, lv[size_t(d)].bound)))
+            return r;
+    hipLaunchKernelGGL(root_place_kernel, dim3(1), dim3(1), 0, st, lv[0].pos, lv[0].B, bad);
     for (int d = 0; d < D; ++d) {
-        Level &p = lv[d];
+        const Level &p = lv[size_t(d)], &c = lv[size_t(d) + 1];
         if (p.bound)
-            hipLaunchKernelGGL(write_nodes_kernel, dim3(grid_for(p.bound)), dim3(kThreads), 0, st, p.mask, p.cnt, p.pos,
-                               p.B, p.large, p.far, int(d == D - 1), words, W, bad);
+            hipLaunchKernelGGL(write_level_kernel, dim3(grid_for(p.bound)), dim3(kThreads), 0, st, LevelArrays(p), p.bound,
+                               LevelArrays(c), d == D - 1 ? leafWord : nullptr, words, W, bad);
     }
-    if (L)
-        hipLaunchKernelGGL(write_leaves_kernel, dim3(grid_for(L)), dim3(kThreads), 0, st, leafWord, L, lv[D].pos, words,
-                           W, bad);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     out.build.leaves = L;
@@ -2519,7 +2542,10 @@ static int mesh_core(Arena &ar, float *dv, int64_t nverts, int has_normals, int3
     if ((r = ar.alloc(segStart, K + 1)) || (r = ar.alloc(segInfo, 2))) return r;
     if (K) {
         hipLaunchKernelGGL(set_u64_kernel, dim3(1), dim3(1), 0, st, segInfo, K);
-        if ((r = run_heads(ar, keys2, segInfo, K, tribits, segInfo + 1, SegmentEmit{segStart}, st))) return r;
+        auto segments = [&](unsigned blocks, const uint64_t *sums) {
+            hipLaunchKernelGGL(segment_emit_kernel, dim3(blocks), dim3(kThreads), 0, st, keys2, segInfo, tribits, sums, segStart);
+        };
+        if ((r = run_heads(ar, keys2, segInfo, K, tribits, segInfo + 1, segments, st))) return r;
         uint64_t info[2];
         if ((r = read_words(segInfo, info, 2, st))) return r;
         V = info[1];

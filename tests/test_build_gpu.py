@@ -545,3 +545,21 @@ def test_mesh_voxels_with_an_empty_word(svo, golden, black, depth):
     assert np.array_equal(t.words(), words) and np.array_equal(t.center(), center)
     assert (t.build_stats()["leaves"] == 0) == (black == 1.0)
     assert t.center()[2] == np.float32(depth) * np.float32(0.5) / np.float32(64)
+
+
+@pytest.mark.parametrize("n", [1, 7, 1023, 1024, 1025, 2047, 2048, 2049, 8191, 8192, 8193, 8200, 16390])
+def test_level_passes_at_tile_edges(svo, golden, n):
+    """Leaf counts around the tiles that the level passes work in, as the first
+    n cells in Morton order from an odd one on (full parents that span two
+    tiles) and as random cells, against the oracle's build."""
+    rng = np.random.default_rng(n)
+    cell = np.arange(32768)
+    z, y, x = (sum(((cell >> (3 * b + a)) & 1) << b for b in range(5)) for a in (2, 1, 0))
+    for name, pick in (("a run", np.arange(3, 3 + n)), ("random", rng.choice(32768, n, replace=False))):
+        vol = np.zeros((32, 32, 32), np.uint32)
+        vol[z[pick], y[pick], x[pick]] = rng.integers(1, 2**32, n, dtype=np.uint32)
+        print(f"[gpu] grid of {n} leaves: {name}", flush=True)
+        t = svo.VoxelOctree.build_from_grid(vol)
+        center, words, _ = orc.build_grid(vol)
+        assert np.array_equal(t.words(), words) and np.array_equal(t.center(), center)
+        assert t.build_stats()["leaves"] == n
