@@ -1000,8 +1000,11 @@ struct BlockParams {
 };
 
 // Voxel on the last slice of an odd-depth cache block: never scanned by
-// VoxelData::buildLowLut (src/VoxelData.cpp:163-166), hence never emitted.
+// VoxelData::buildLowLut (src/VoxelData.cpp:163-166), hence never emitted. Blocks
+// of edge 2 have no node of their own in that table (its cells are of edge 2, and
+// a block's own occupancy is the top table's): nothing is left out there.
 __device__ __forceinline__ bool unscanned(uint32_t z, const BlockParams &bp) {
+    if (bp.cacheLog == 1) return false;
     const int z0 = int(z >> bp.cacheLog) << bp.cacheLog;
     const int bd = min(bp.cache, bp.data[2] - z0);
     return (bd & 1) && int(z) == z0 + bd - 1;
@@ -2107,8 +2110,8 @@ int finish_leaves(Arena &ar, const Geometry &g, uint64_t *key, uint32_t *word, u
     };
     // an odd depth has a last slice that is not scanned: its voxels, if any,
     // are dropped, so the prefix sum is under way before the counts are read
-    // (waiting for them first took a 321x301x283 grid from 1.84 ms to 1.87)
-    const bool likely = V && (g.dataD & 1);
+    // (waiting for them first took a 203x251x189 grid from 1.84 ms to 1.87)
+    const bool likely = V && (g.dataD & 1) && g.cacheLog != 1;
     if (likely && ((r = ar.alloc(keep, V)) || (r = ar.alloc(at, V)))) return r;
     flags();
     if (mesh && nBlocks > 1)

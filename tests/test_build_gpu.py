@@ -563,3 +563,30 @@ def test_level_passes_at_tile_edges(svo, golden, n):
         center, words, _ = orc.build_grid(vol)
         assert np.array_equal(t.words(), words) and np.array_equal(t.center(), center)
         assert t.build_stats()["leaves"] == n
+
+
+@pytest.mark.parametrize("shape,mem", [((1, 2, 2), 1 << 30), ((3, 4, 4), 100), ((1, 3, 3), 100), ((5, 8, 7), 200)])
+def test_grid_last_slice_of_smallest_blocks(svo, golden, shape, mem):
+    """Odd depths in cache blocks of edge 2, whose last slice is emitted like
+    any other, against the oracle's build."""
+    vol = np.random.default_rng(3).integers(1, 2**32, shape, dtype=np.uint32)
+    print(f"[gpu] grid {shape} mem={mem}", flush=True)
+    t = svo.VoxelOctree.build_from_grid(vol, memory_budget=mem)
+    center, words, _ = orc.build_grid(vol, mem)
+    assert np.array_equal(t.words(), words) and np.array_equal(t.center(), center)
+
+
+@pytest.mark.parametrize("depth", [6, 7, 8])
+def test_mesh_last_slice_of_smallest_blocks(svo, golden, depth):
+    """The same for a mesh, which fills its last slice."""
+    rng = np.random.default_rng(29)
+    v = rng.random((60, 3)).astype(np.float32)
+    v[:2] = [[0, 0, 0], [1, 1, 1]]
+    v[:, 2] *= 1.0 if depth == 8 else (depth - 2 + 0.5) / 6
+    tab = np.zeros((60, 9), np.float32)
+    tab[:, :3], tab[:, 6:] = v, 200.0
+    counts, idx = np.full(20, 3, np.int32), np.arange(60, dtype=np.int32)
+    print(f"[gpu] mesh 8^3, depth {depth}, mem=200", flush=True)
+    t = svo.VoxelOctree.build_from_mesh(tab, False, counts, idx, 8, threads=1, memory_budget=200)
+    center, words, _ = orc.Mesh(tab, False, counts, idx).build(8, 1, 200)
+    assert np.array_equal(t.words(), words) and np.array_equal(t.center(), center)
