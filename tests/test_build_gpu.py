@@ -590,3 +590,20 @@ def test_mesh_last_slice_of_smallest_blocks(svo, golden, depth):
     t = svo.VoxelOctree.build_from_mesh(tab, False, counts, idx, 8, threads=1, memory_budget=200)
     center, words, _ = orc.Mesh(tab, False, counts, idx).build(8, 1, 200)
     assert np.array_equal(t.words(), words) and np.array_equal(t.center(), center)
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 2), (7, 3, 5), (8, 16, 16), (9, 16, 17), (50, 40, 33), (16, 32, 64), (15, 32, 64),
+                                   (64, 16, 16), (2, 100, 100), (131, 130, 129)])
+@pytest.mark.parametrize("fill", [0.0, 0.3, 1.0])
+def test_grid_shapes(svo, golden, shape, fill):
+    """Dense grids of edge shapes, those gone through in their bounding cube's
+    Morton order and the flatter ones that are sorted, empty to full, against
+    the oracle's build."""
+    rng = np.random.default_rng(5)
+    vol = rng.integers(1, 2**32, shape, dtype=np.uint32)
+    vol[rng.random(shape) >= fill] = 0
+    print(f"[gpu] grid {shape} filled to {fill}", flush=True)
+    t = svo.VoxelOctree.build_from_grid(vol)
+    center, words, _ = orc.build_grid(vol)
+    assert np.array_equal(t.words(), words) and np.array_equal(t.center(), center)
+    assert t.build_stats()["candidates"] == np.count_nonzero(vol)
