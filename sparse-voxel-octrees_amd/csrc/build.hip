@@ -62,7 +62,7 @@ constexpr int kThreads = 256;
 // rocPRIM sorts arrays below this size by merging, two launches per doubling
 // above 1024 items (20 launches for the 480 K candidates of a 256^3 mesh);
 // from here up its radix passes (one per 8 key bits, three or so) are faster.
-// 256^3 mesh build 1.12 -> 1.03 ms, a 203x251x189 volume 2.18 -> 2.10 ms;
+// 256^3 mesh build 1.12 -> 1.03 ms;
 // with the line at 2^12 or 2^14 a 64^3 mesh (30 K candidates) took 0.85
 // instead of 0.75 ms. The default line is 2^20.
 using SortConfig = rocprim::radix_sort_config<rocprim::default_config, rocprim::default_config, rocprim::default_config,
@@ -1431,14 +1431,26 @@ __global__ void terrain_words_kernel(const uint64_t *__restrict__ key, uint64_t 
 // exclusive prefix sums with the element count in device memory
 // ---------------------------------------------------------------------------
 
-// Three passes over blocks of kScanTile elements: per-block sums, one
-// workgroup scanning the block sums (and writing the grand total), then each
-// block's scan plus its offset. The count is read on the device, so a pass
+// Passes over blocks of kScanTile elements: per-block sums, then each block's
+// scan plus the sum of the blocks before it. Up to kDirectTiles blocks, each
+// block of the last pass adds up the sums before its own; above, a workgroup of
+// its own scans them in between. The count may be read on the device, so a pass
 // whose input count was produced by an earlier kernel needs no round trip to
 // the host; grids are sized by a host-side upper bound and blocks past the
-// count exit at once.
+// count have nothing to do.
 constexpr int kScanItems = 8;
 constexpr uint64_t kScanTile = uint64_t(kThreads) * kScanItems;
+
+struct Count {  // on the device, or known to the host
+    const uint64_t *dev = nullptr;
+    uint64_t n = 0;
+    __device__ uint64_t get() const { return dev ? *dev : n; }
+};
+
+struct TileSums {
+    uint64_t *sums, *total;  // per block, scanned or not; their grand total (total may be null)
+    bool scanned;
+};
 
 // Exclusive sum of `v` over the Threads threads of the workgroup (lds holds
 // Threads / 64 words); *all = total.
@@ -1464,6 +1476,17 @@ __device__ __forceinline__ uint64_t block_exclusive(uint64_t v, uint64_t *lds, u
     return before + x - v;
 }
 
+// Sum of the blocks before this one; the last block also writes the total.
+// Every thread of the workgroup calls it.
+__device__ __forceinline__ uint64_t tile_offset(const TileSums &t, uint64_t *lds) {
+    if (t.scanned) return t.sums[blockIdx.x];
+    uint64_t before = 0, all;
+    for (uint32_t i = threadIdx.x; i < blockIdx.x; i += kThreads) before += t.sums[i];
+    block_exclusive(before, lds, &all);
+    if (t.total && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *t.total = all + t.sums[blockIdx.x];
+    return all;
+}
+
 // Thread items [first, first + kScanItems) of in[0, n) (0 past n); a full
 // run of 32-bit items is two 16-byte loads (the arrays are 16-byte aligned).
 template <typename In>
@@ -1483,10 +1506,10 @@ __device__ __forceinline__ void load_items(const In *__restrict__ in, uint64_t f
 }
 
 template <typename In>
-__global__ void __launch_bounds__(kThreads) scan_sums_kernel(const In *__restrict__ in, const uint64_t *__restrict__ nptr,
+__global__ void __launch_bounds__(kThreads) scan_sums_kernel(const In *__restrict__ in, Count count,
                                                              uint64_t *__restrict__ sums) {
     __shared__ uint64_t lds[kThreads / 64];
-    const uint64_t n = *nptr;
+    const uint64_t n = count.get();
     const uint64_t base = uint64_t(blockIdx.x) * kScanTile;
     if (base >= n) {
         if (threadIdx.x == 0) sums[blockIdx.x] = 0;
@@ -1527,15 +1550,18 @@ __global__ void __launch_bounds__(kSumThreads) scan_block_sums_kernel(uint64_t *
         }
         carry += all;
     }
-    if (threadIdx.x == 0) *total = carry;
+    if (total && threadIdx.x == 0) *total = carry;
 }
 
+// close: out[n] = the total.
 template <typename In>
-__global__ void __launch_bounds__(kThreads) scan_down_kernel(const In *__restrict__ in, const uint64_t *__restrict__ nptr,
-                                                             const uint64_t *__restrict__ offs, uint64_t *__restrict__ out) {
+__global__ void __launch_bounds__(kThreads) scan_down_kernel(const In *__restrict__ in, Count count, TileSums t, bool close,
+                                                             uint64_t *__restrict__ out) {
     __shared__ uint64_t lds[kThreads / 64];
-    const uint64_t n = *nptr;
+    const uint64_t n = count.get();
     const uint64_t base = uint64_t(blockIdx.x) * kScanTile;
+    const uint64_t offset = tile_offset(t, lds);
+    if (close && blockIdx.x == 0 && threadIdx.x == 0 && n == 0) out[0] = 0;
     if (base >= n) return;
     const uint64_t first = base + uint64_t(threadIdx.x) * kScanItems;
     uint64_t v[kScanItems];
@@ -1544,7 +1570,8 @@ __global__ void __launch_bounds__(kThreads) scan_down_kernel(const In *__restric
 #pragma unroll
     for (int k = 0; k < kScanItems; ++k) sum += v[k];
     uint64_t total;
-    uint64_t run = offs[blockIdx.x] + block_exclusive(sum, lds, &total);
+    uint64_t run = offset + block_exclusive(sum, lds, &total);
+    if (close && threadIdx.x == 0 && base + kScanTile >= n) out[n] = offset + total;
     if (first + kScanItems <= n) {
         // a full run: four 16-byte stores
         uint64_t o[kScanItems];
@@ -1623,10 +1650,9 @@ __device__ __forceinline__ uint32_t tile_heads(const uint64_t bits[kScanItems], 
 }
 
 __global__ void __launch_bounds__(kThreads) run_sums_kernel(const uint64_t *__restrict__ keys,
-                                                            const uint64_t *__restrict__ nptr, int shift,
-                                                            uint64_t *__restrict__ sums) {
+                                                            Count counted, int shift, uint64_t *__restrict__ sums) {
     __shared__ uint32_t part[kThreads / 64];
-    const uint64_t n = *nptr;
+    const uint64_t n = counted.get();
     const uint64_t base = uint64_t(blockIdx.x) * kScanTile;
     if (base >= n) {
         if (threadIdx.x == 0) sums[blockIdx.x] = 0;
@@ -1646,21 +1672,20 @@ __global__ void __launch_bounds__(kThreads) run_sums_kernel(const uint64_t *__re
     }
 }
 
-// The fold's segments: segStart[j] = the first candidate of voxel j.
-__global__ void __launch_bounds__(kThreads) segment_emit_kernel(const uint64_t *__restrict__ keys,
-                                                                const uint64_t *__restrict__ nptr, int shift,
-                                                                const uint64_t *__restrict__ offs,
-                                                                uint64_t *__restrict__ segStart) {
+// The fold's segments: segStart[j] = the first candidate of voxel j, closed by
+// the candidate count.
+__global__ void __launch_bounds__(kThreads) segment_emit_kernel(const uint64_t *__restrict__ keys, uint64_t n, int shift,
+                                                                TileSums t, uint64_t *__restrict__ segStart) {
     __shared__ uint16_t head[kScanTile];
     __shared__ uint32_t at[kScanItems * kThreads / 64];
-    const uint64_t n = *nptr;
+    __shared__ uint64_t lds[kThreads / 64];
     const uint64_t base = uint64_t(blockIdx.x) * kScanTile;
-    if (base >= n) return;
+    const uint64_t j = tile_offset(t, lds);
     uint64_t bits[kScanItems];
     tile_flags(keys, base, n, shift, bits, nullptr);
     const uint32_t heads = tile_heads(bits, head, at);
-    const uint64_t j = offs[blockIdx.x];
     for (uint32_t h = threadIdx.x; h < heads; h += kThreads) segStart[j + h] = base + head[h];
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) segStart[j + heads] = n;
 }
 
 // Voxels of a dense grid in Morton order: a workgroup takes kScanTile
@@ -1726,22 +1751,22 @@ __global__ void __launch_bounds__(kThreads) brick_emit_kernel(const uint32_t *__
 // child mask and subtree size (its children, at most 8 since keys are unique,
 // follow the head). Leaves have no sizes.
 template <bool Leaves>
-__global__ void __launch_bounds__(kThreads) parent_emit_kernel(LevelArrays child, LevelArrays p,
-                                                               const uint64_t *__restrict__ offs) {
+__global__ void __launch_bounds__(kThreads) parent_emit_kernel(LevelArrays child, LevelArrays p, TileSums t) {
     __shared__ uint64_t key[kScanTile + 8], size[Leaves ? 1 : kScanTile + 8];
     __shared__ uint16_t head[kScanTile];
     __shared__ uint32_t at[kScanItems * kThreads / 64];
+    __shared__ uint64_t lds[kThreads / 64];
     const uint64_t n = *child.cnt;
     const uint64_t base = uint64_t(blockIdx.x) * kScanTile;
+    const uint64_t j = tile_offset(t, lds);
     if (base >= n) return;
     uint64_t bits[kScanItems];
     tile_flags(child.key, base, n, 3, bits, key);
-    for (uint64_t t = threadIdx.x; t < 8; t += kThreads)
-        if (base + kScanTile + t < n) key[kScanTile + t] = child.key[base + kScanTile + t];
+    if (threadIdx.x < 8 && base + kScanTile + threadIdx.x < n)
+        key[kScanTile + threadIdx.x] = child.key[base + kScanTile + threadIdx.x];
     if constexpr (!Leaves)
-        for (uint64_t t = threadIdx.x; t < kScanTile + 8; t += kThreads) size[t] = base + t < n ? child.S[base + t] : 0;
+        for (uint64_t q = threadIdx.x; q < kScanTile + 8; q += kThreads) size[q] = base + q < n ? child.S[base + q] : 0;
     const uint32_t heads = tile_heads(bits, head, at);
-    const uint64_t j = offs[blockIdx.x];
     for (uint32_t h = threadIdx.x; h < heads; h += kThreads) {
         const uint32_t i = head[h];
         const uint64_t parent = key[i] >> 3;
@@ -1782,58 +1807,62 @@ __global__ void widen_u32_kernel(const uint32_t *src, uint64_t *dst) { *dst = *s
 // host helpers
 // ---------------------------------------------------------------------------
 
-// Exclusive prefix sum of in[0, n) into out (64-bit), n read from the device
-// word *nptr; `bound` (host) is an upper bound of n that sizes the grids.
-// *total (device, may be null) receives the sum of all n elements.
+// Blocks up to which the last pass adds up the block sums itself. A block then
+// reads up to 8 KB of sums that are in cache, where the pass in between is a
+// launch and one workgroup's work, on every scan and level of a small build: a
+// 256^3 mesh 950 us with it, 840 without, a 64^3 one 650 and 557, a 700^3 one
+// 2,565 and 2,490. Above, the sums read grow with the square of the blocks (24 M
+// keys: 11.5 K blocks, 0.5 GB) while the pass stays at 14 us.
+constexpr uint64_t kDirectTiles = 1024;
+
+// The block sums of `bound` elements; `scan_sums` runs between the two passes.
+int tile_sums(Arena &ar, uint64_t bound, uint64_t *total, TileSums &t, unsigned &nb) {
+    const uint64_t blocks = std::max<uint64_t>(1, (bound + kScanTile - 1) / kScanTile);
+    if (blocks > 0x7FFFFFFFull) return fail(SVO_ERR_LIMIT, "builder: scan too large");
+    nb = unsigned(blocks);
+    t.total = total;
+    t.scanned = blocks > kDirectTiles;
+    return ar.alloc(t.sums, blocks);
+}
+void scan_sums(const TileSums &t, unsigned nb, hipStream_t s) {
+    if (t.scanned)
+        hipLaunchKernelGGL(scan_block_sums_kernel, dim3(1), dim3(kSumThreads), 0, s, t.sums, uint64_t(nb), t.total);
+}
+
+// Exclusive prefix sum of in[0, n) into out (64-bit); *total (device, may be
+// null) receives the sum of all n elements, and out[n] too with `close`.
 template <typename In>
-int exclusive_scan_dev(Arena &ar, const In *in, uint64_t *out, const uint64_t *nptr, uint64_t bound, uint64_t *total,
-                       hipStream_t s) {
-    const uint64_t nb = std::max<uint64_t>(1, (bound + kScanTile - 1) / kScanTile);
-    if (nb > 0x7FFFFFFFull) return fail(SVO_ERR_LIMIT, "builder: scan too large");
+int exclusive_scan(Arena &ar, const In *in, uint64_t *out, uint64_t n, hipStream_t s, uint64_t *total = nullptr,
+                   bool close = false) {
     if (reinterpret_cast<uintptr_t>(in) % 16 || reinterpret_cast<uintptr_t>(out) % 16)
         return fail(SVO_ERR_DEVICE, "builder: scan arrays must be 16-byte aligned (internal error)");
-    uint64_t *sums, *tot = total;
-    int r = ar.alloc(sums, nb);
-    if (r) return r;
-    if (!tot && (r = ar.alloc(tot, 1))) return r;
-    hipLaunchKernelGGL(scan_sums_kernel<In>, dim3(unsigned(nb)), dim3(kThreads), 0, s, in, nptr, sums);
-    hipLaunchKernelGGL(scan_block_sums_kernel, dim3(1), dim3(kSumThreads), 0, s, sums, nb, tot);
-    hipLaunchKernelGGL(scan_down_kernel<In>, dim3(unsigned(nb)), dim3(kThreads), 0, s, in, nptr, sums, out);
+    TileSums t;
+    unsigned nb;
+    if (int r = tile_sums(ar, n, total, t, nb)) return r;
+    const Count count{nullptr, n};
+    hipLaunchKernelGGL(scan_sums_kernel<In>, dim3(nb), dim3(kThreads), 0, s, in, count, t.sums);
+    scan_sums(t, nb, s);
+    hipLaunchKernelGGL(scan_down_kernel<In>, dim3(nb), dim3(kThreads), 0, s, in, count, t, close, out);
     HIP_TRY(hipGetLastError());
-    ar.release(sums);
-    if (!total) ar.release(tot);
+    ar.release(t.sums);
     return SVO_OK;
 }
 
-// Run heads of keys[0, *nptr) (sorted; runs of equal keys >> shift): each
-// tile's heads before it in sums[], which emit(blocks, sums) reads; *total
-// (device) = the head count. `bound` (host) bounds *nptr and sizes the grids.
+// Run heads of keys[0, count) (sorted; runs of equal keys >> shift): each
+// tile's heads in t, with which emit(blocks, t) goes on; *total (device) = the
+// head count. `bound` (host) bounds the count and sizes the grids.
 template <typename Emit>
-int run_heads(Arena &ar, const uint64_t *keys, const uint64_t *nptr, uint64_t bound, int shift, uint64_t *total,
-              const Emit &emit, hipStream_t s) {
-    const uint64_t nb = std::max<uint64_t>(1, (bound + kScanTile - 1) / kScanTile);
-    if (nb > 0x7FFFFFFFull) return fail(SVO_ERR_LIMIT, "builder: scan too large");
-    uint64_t *sums;
-    int r = ar.alloc(sums, nb);
-    if (r) return r;
-    hipLaunchKernelGGL(run_sums_kernel, dim3(unsigned(nb)), dim3(kThreads), 0, s, keys, nptr, shift, sums);
-    hipLaunchKernelGGL(scan_block_sums_kernel, dim3(1), dim3(kSumThreads), 0, s, sums, nb, total);
-    emit(unsigned(nb), sums);
+int run_heads(Arena &ar, const uint64_t *keys, Count count, uint64_t bound, int shift, uint64_t *total, const Emit &emit,
+              hipStream_t s) {
+    TileSums t;
+    unsigned nb;
+    if (int r = tile_sums(ar, bound, total, t, nb)) return r;
+    hipLaunchKernelGGL(run_sums_kernel, dim3(nb), dim3(kThreads), 0, s, keys, count, shift, t.sums);
+    scan_sums(t, nb, s);
+    emit(nb, t);
     HIP_TRY(hipGetLastError());
-    ar.release(sums);
+    ar.release(t.sums);
     return SVO_OK;
-}
-
-// The same with a host-known count; *total (device, may be null) as above.
-template <typename In>
-int exclusive_scan(Arena &ar, const In *in, uint64_t *out, uint64_t n, hipStream_t s, uint64_t *total = nullptr) {
-    uint64_t *nd;
-    int r = ar.alloc(nd, 1);
-    if (r) return r;
-    hipLaunchKernelGGL(set_u64_kernel, dim3(1), dim3(1), 0, s, nd, n);
-    r = exclusive_scan_dev(ar, in, out, nd, n, total, s);
-    ar.release(nd);
-    return r;
 }
 
 // Reads device words into host values in one copy (one round trip).
@@ -1843,16 +1872,16 @@ int read_words(const uint64_t *src, uint64_t *dst, int count, hipStream_t s) {
     return SVO_OK;
 }
 
-// Exclusive scan with a host-known count whose total the host needs next.
+// Exclusive scan whose total the host needs next.
 template <typename In>
-int scan_count(Arena &ar, const In *in, uint64_t *out, uint64_t n, hipStream_t s, uint64_t &total) {
+int scan_count(Arena &ar, const In *in, uint64_t *out, uint64_t n, hipStream_t s, uint64_t &total, bool close = false) {
     if (n == 0) {
         total = 0;
         return SVO_OK;
     }
     uint64_t *tot;
     int r = ar.alloc(tot, 1);
-    if (r || (r = exclusive_scan(ar, in, out, n, s, tot)) || (r = read_words(tot, &total, 1, s))) return r;
+    if (r || (r = exclusive_scan(ar, in, out, n, s, tot, close)) || (r = read_words(tot, &total, 1, s))) return r;
     ar.release(tot);
     return SVO_OK;
 }
@@ -2048,11 +2077,11 @@ int emit_tree(Arena &ar, const Geometry &g, uint64_t *leafKey, uint32_t *leafWor
             p.bound = d < 21 ? std::min(c.bound, uint64_t(1) << (3 * d)) : c.bound;
             if ((r = level_arrays(p, d == 0))) return r;
             // every parent below the count is written once (by its first child)
-            auto parents = [&](unsigned blocks, const uint64_t *sums) {
+            auto parents = [&](unsigned blocks, const TileSums &t) {
                 auto kernel = d == D - 1 ? parent_emit_kernel<true> : parent_emit_kernel<false>;
-                hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), 0, st, LevelArrays(c), LevelArrays(p), sums);
+                hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), 0, st, LevelArrays(c), LevelArrays(p), t);
             };
-            if ((r = run_heads(ar, c.key, c.cnt, c.bound, 3, p.cnt, parents, st))) return r;
+            if ((r = run_heads(ar, c.key, Count{c.cnt, 0}, c.bound, 3, p.cnt, parents, st))) return r;
         }
         ar.release(c.key);
         HIP_TRY(hipGetLastError());
@@ -2538,8 +2567,7 @@ static int mesh_core(Arena &ar, float *dv, int64_t nverts, int has_normals, int3
                            boxes);
     HIP_TRY(hipGetLastError());
     uint64_t R;
-    if ((r = scan_count(ar, rows, rowStart, P, st, R))) return r;
-    hipLaunchKernelGGL(set_u64_kernel, dim3(1), dim3(1), 0, st, rowStart + P, R);
+    if ((r = scan_count(ar, rows, rowStart, P, st, R, true))) return r;
     ar.release(rows);
     // each row's pair (the row passes read it instead of searching rowStart)
     if ((r = ar.alloc(rowPair, R))) return r;
@@ -2601,19 +2629,17 @@ static int mesh_core(Arena &ar, float *dv, int64_t nverts, int has_normals, int3
     uint64_t *segStart, *vkey, *segInfo;
     uint32_t *vword;
     uint8_t *vcount;
-    if ((r = ar.alloc(segStart, K + 1)) || (r = ar.alloc(segInfo, 2))) return r;
+    if ((r = ar.alloc(segStart, K + 1)) || (r = ar.alloc(segInfo, 1))) return r;
     if (K) {
-        hipLaunchKernelGGL(set_u64_kernel, dim3(1), dim3(1), 0, st, segInfo, K);
-        auto segments = [&](unsigned blocks, const uint64_t *sums) {
-            hipLaunchKernelGGL(segment_emit_kernel, dim3(blocks), dim3(kThreads), 0, st, keys2, segInfo, tribits, sums, segStart);
+        auto segments = [&](unsigned blocks, const TileSums &t) {
+            hipLaunchKernelGGL(segment_emit_kernel, dim3(blocks), dim3(kThreads), 0, st, keys2, K, tribits, t, segStart);
         };
-        if ((r = run_heads(ar, keys2, segInfo, K, tribits, segInfo + 1, segments, st))) return r;
-        uint64_t info[2];
-        if ((r = read_words(segInfo, info, 2, st))) return r;
-        V = info[1];
+        if ((r = run_heads(ar, keys2, Count{nullptr, K}, K, tribits, segInfo, segments, st))) return r;
+        if ((r = read_words(segInfo, &V, 1, st))) return r;
+    } else {
+        hipLaunchKernelGGL(set_u64_kernel, dim3(1), dim3(1), 0, st, segStart, uint64_t(0));
     }
     ar.release(segInfo);
-    hipLaunchKernelGGL(set_u64_kernel, dim3(1), dim3(1), 0, st, segStart + V, K);
     if (sink) return write_volume(ar, g, mp, tribits, keys2, segStart, V, pos, nrm, col, sliceZ, sink->fp);
     if ((r = ar.alloc(vkey, V)) || (r = ar.alloc(vword, V)) || (r = ar.alloc(vcount, V))) return r;
     if (V) {
@@ -3009,16 +3035,17 @@ int build_grid(const uint32_t *grid, int w, int h, int d, const svo_build_opts *
     uint64_t V, *key;
     uint32_t *word;
     if (const uint64_t cells = uint64_t(1) << (3 * g.depth); cells / kCubeShare <= N) {
-        const uint64_t nb = std::max<uint64_t>(1, cells / kScanTile);
-        if (nb > 0x7FFFFFFFull) return fail(SVO_ERR_LIMIT, "builder: scan too large");
-        uint64_t *sums, *total;
-        if ((r = ar.alloc(sums, nb)) || (r = ar.alloc(total, 1))) return r;
-        hipLaunchKernelGGL(brick_sums_kernel, dim3(unsigned(nb)), dim3(kThreads), 0, st, dg, w, h, d, sums);
-        hipLaunchKernelGGL(scan_block_sums_kernel, dim3(1), dim3(kSumThreads), 0, st, sums, nb, total);
+        uint64_t *total;
+        TileSums t;
+        unsigned nb;
+        if ((r = ar.alloc(total, 1)) || (r = tile_sums(ar, cells, total, t, nb))) return r;
+        t.scanned = true;  // the total is needed before the second pass
+        hipLaunchKernelGGL(brick_sums_kernel, dim3(nb), dim3(kThreads), 0, st, dg, w, h, d, t.sums);
+        scan_sums(t, nb, st);
         if ((r = read_words(total, &V, 1, st)) || (r = ar.alloc(key, V)) || (r = ar.alloc(word, V))) return r;
-        hipLaunchKernelGGL(brick_emit_kernel, dim3(unsigned(nb)), dim3(kThreads), 0, st, dg, w, h, d, sums, key, word);
+        hipLaunchKernelGGL(brick_emit_kernel, dim3(nb), dim3(kThreads), 0, st, dg, w, h, d, t.sums, key, word);
         HIP_TRY(hipGetLastError());
-        ar.release(sums);
+        ar.release(t.sums);
         ar.release(total);
     } else {
         uint32_t *flag, *word0;

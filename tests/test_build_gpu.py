@@ -607,3 +607,14 @@ def test_grid_shapes(svo, golden, shape, fill):
     center, words, _ = orc.build_grid(vol)
     assert np.array_equal(t.words(), words) and np.array_equal(t.center(), center)
     assert t.build_stats()["candidates"] == np.count_nonzero(vol)
+
+
+@pytest.mark.parametrize("width", [127, 128, 129])
+def test_level_passes_at_the_largest_direct_scan(svo, golden, width):
+    """Leaf counts below, at and above the 1024 tiles of 2048 up to which a
+    pass adds up the tile sums before its own, against the oracle's build."""
+    vol = np.random.default_rng(11).integers(1, 2**32, (128, 128, width), dtype=np.uint32)
+    print(f"[gpu] grid of {vol.size} leaves", flush=True)
+    t = svo.VoxelOctree.build_from_grid(vol)
+    center, words, _ = orc.build_grid(vol)
+    assert np.array_equal(t.words(), words) and np.array_equal(t.center(), center)
