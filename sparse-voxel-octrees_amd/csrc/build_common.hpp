@@ -145,6 +145,74 @@ __device__ __forceinline__ bool tri_box(const float c[3], const float h[3], cons
     return nrm[0] * vmax[0] + nrm[1] * vmax[1] + nrm[2] * vmax[2] >= 0.0f;
 }
 
+// tri_box for the voxels of one row, whose centres differ in x only: the same
+// expressions on the same values, those without an x taken once. That is the
+// three tests about the x axis and the box's y and z extents, which also rule
+// out whole rows; the six other axis tests, the x extent and the plane remain
+// per voxel, without a branch between them. A mesh's vertices lie in the unit
+// cube by then, so nothing here is a NaN and minimum and maximum stand for the
+// comparisons they are made of.
+struct TriRow {
+    float v0[3], v1[3], v2[3], e0[3], e1[3], e2[3], tx[3];  // [0] per voxel, x from tx
+    float h[3], n0;
+    bool out;
+
+    static __device__ __forceinline__ bool apart(float pa, float pb, float rad) {
+        return (fminf(pa, pb) > rad) | (fmaxf(pa, pb) < -rad);
+    }
+    __device__ __forceinline__ bool wide(int k) const {
+        return (fminf(fminf(v0[k], v1[k]), v2[k]) > h[k]) | (fmaxf(fmaxf(v0[k], v1[k]), v2[k]) < -h[k]);
+    }
+    __device__ __forceinline__ TriRow(float cy, float cz, const float half[3], const float tv[9]) {
+        const float c[3] = {0.0f, cy, cz};
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            h[k] = half[k];
+            tx[k] = tv[3 * k];
+            if (k == 0) continue;
+            v0[k] = tv[k] - c[k];
+            v1[k] = tv[3 + k] - c[k];
+            v2[k] = tv[6 + k] - c[k];
+            e0[k] = v1[k] - v0[k];
+            e1[k] = v2[k] - v1[k];
+            e2[k] = v0[k] - v2[k];
+        }
+        out = wide(1) | wide(2);
+        out |= apart(e0[2] * v0[1] - e0[1] * v0[2], e0[2] * v2[1] - e0[1] * v2[2], fabsf(e0[2]) * h[1] + fabsf(e0[1]) * h[2]);
+        out |= apart(e1[2] * v0[1] - e1[1] * v0[2], e1[2] * v2[1] - e1[1] * v2[2], fabsf(e1[2]) * h[1] + fabsf(e1[1]) * h[2]);
+        out |= apart(e2[2] * v0[1] - e2[1] * v0[2], e2[2] * v1[1] - e2[1] * v1[2], fabsf(e2[2]) * h[1] + fabsf(e2[1]) * h[2]);
+        n0 = e0[1] * e1[2] - e0[2] * e1[1];
+    }
+    __device__ __forceinline__ bool hit(float cx) {
+        v0[0] = tx[0] - cx;
+        v1[0] = tx[1] - cx;
+        v2[0] = tx[2] - cx;
+        e0[0] = v1[0] - v0[0];
+        e1[0] = v2[0] - v1[0];
+        e2[0] = v0[0] - v2[0];
+        bool sep = wide(0);
+        float fx = fabsf(e0[0]);
+        sep |= apart(-e0[2] * v0[0] + e0[0] * v0[2], -e0[2] * v2[0] + e0[0] * v2[2], fabsf(e0[2]) * h[0] + fx * h[2]);
+        sep |= apart(e0[1] * v1[0] - e0[0] * v1[1], e0[1] * v2[0] - e0[0] * v2[1], fabsf(e0[1]) * h[0] + fx * h[1]);
+        fx = fabsf(e1[0]);
+        sep |= apart(-e1[2] * v0[0] + e1[0] * v0[2], -e1[2] * v2[0] + e1[0] * v2[2], fabsf(e1[2]) * h[0] + fx * h[2]);
+        sep |= apart(e1[1] * v0[0] - e1[0] * v0[1], e1[1] * v1[0] - e1[0] * v1[1], fabsf(e1[1]) * h[0] + fx * h[1]);
+        fx = fabsf(e2[0]);
+        sep |= apart(-e2[2] * v0[0] + e2[0] * v0[2], -e2[2] * v1[0] + e2[0] * v1[2], fabsf(e2[2]) * h[0] + fx * h[2]);
+        sep |= apart(e2[1] * v1[0] - e2[0] * v1[1], e2[1] * v2[0] - e2[0] * v2[1], fabsf(e2[1]) * h[0] + fx * h[1]);
+        const float nrm[3] = {n0, e0[2] * e1[0] - e0[0] * e1[2], e0[0] * e1[1] - e0[1] * e1[0]};
+        float vmin[3], vmax[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const float a = -h[k] - v0[k], b = h[k] - v0[k];
+            vmin[k] = nrm[k] > 0.0f ? a : b;
+            vmax[k] = nrm[k] > 0.0f ? b : a;
+        }
+        sep |= nrm[0] * vmin[0] + nrm[1] * vmin[1] + nrm[2] * vmin[2] > 0.0f;
+        return !sep & (nrm[0] * vmax[0] + nrm[1] * vmax[1] + nrm[2] * vmax[2] >= 0.0f);
+    }
+};
+
 __device__ __forceinline__ void cross3(const float a[3], const float b[3], float r[3]) {
     r[0] = a[1] * b[2] - a[2] * b[1];
     r[1] = a[2] * b[0] - a[0] * b[2];

@@ -618,3 +618,20 @@ def test_level_passes_at_the_largest_direct_scan(svo, golden, width):
     t = svo.VoxelOctree.build_from_grid(vol)
     center, words, _ = orc.build_grid(vol)
     assert np.array_equal(t.words(), words) and np.array_equal(t.center(), center)
+
+
+@pytest.mark.parametrize("res,extent,threads", [(1024, (0.01, 1, 1), 1), (300, (1, 0.3, 0.02), 1), (66, (1, 0.5, 0.5), 1),
+                                                (67, (1, 0.5, 0.5), 1), (68, (1, 0.5, 0.5), 1)])
+def test_rows_of_large_triangles(svo, golden, res, extent, threads):
+    """Triangles over the whole volume: a million rows of a few voxels, rows
+    of hundreds, and rows around the 64 voxels that a row's mark holds,
+    against the oracle's build."""
+    v = np.array([[0, 0, 0], [1, 1, 0.3], [0.2, 0.9, 1], [1, 0, 1], [0, 0.5, 0.2], [0.4, 1, 1],
+                  [0.1, 0.1, 0.9], [1, 0.2, 0.8], [0.6, 0.9, 0]], np.float32) * np.float32(extent)
+    tab = np.zeros((9, 9), np.float32)
+    tab[:, :3], tab[:, 6:] = v, 150.0
+    counts, idx = np.full(3, 3, np.int32), np.arange(9, dtype=np.int32)
+    print(f"[gpu] three large triangles at {res}, extent {extent}", flush=True)
+    t = svo.VoxelOctree.build_from_mesh(tab, False, counts, idx, res, threads=threads, memory_budget=1 << 30)
+    center, words, _ = orc.Mesh(tab, False, counts, idx).build(res, threads, 1 << 30)
+    assert np.array_equal(t.words(), words) and np.array_equal(t.center(), center)
