@@ -60,7 +60,7 @@ using namespace dev;
 constexpr int kThreads = 256;
 
 // rocPRIM sorts arrays below this size by merging, two launches per doubling
-// above 1024 items (20 launches for the 480 K candidates of a 256^3 mesh);
+// above 1024 items (20 launches for the 600 K candidates of a 256^3 mesh);
 // from here up its radix passes (one per 8 key bits, three or so) are faster.
 // 256^3 mesh build 1.12 -> 1.03 ms;
 // with the line at 2^12 or 2^14 a 64^3 mesh (30 K candidates) took 0.85
@@ -798,9 +798,9 @@ __device__ __forceinline__ void fold_voxel(const uint64_t *__restrict__ keys, ui
 // counts differ (one lane per voxel would run every lane as long as the
 // voxel with the most triangles). Volumes too small for kFoldWaves waves of 512
 // voxels (8 per SIMD) take fewer per wave, down to one per lane: at 512 a
-// 256^3 mesh's 0.1 M voxels gave 4 in 5 SIMDs no wave, and each wave 8 or more
+// 256^3 mesh's 0.3 M voxels gave 4 in 9 SIMDs no wave, and each wave 8 or more
 // rounds of dependent loads: 72 us of a 1,107 us build, now 1,061; a 64^3 one
-// 818 -> 776; 2048^3 has 18 K waves either way (0.87 ms, bound by its VALU work).
+// 818 -> 776; 2048^3 has 38 K waves either way (0.87 ms, bound by its VALU work).
 constexpr uint64_t kFoldChunk = 512, kFoldWaves = 8192;
 inline uint64_t fold_chunk(uint64_t S) {
     return std::min(kFoldChunk, std::max<uint64_t>(64, (S / kFoldWaves + 63) / 64 * 64));
@@ -1448,8 +1448,8 @@ struct Row {
 //
 // The passes move 12 bytes per row and then 12 and its keys (the pair's box
 // stays in cache), a third of what they did with a 24-byte record per row and
-// counts and 64-bit offsets from a prefix sum over all rows: a 2048^3 mesh (18 M
-// rows, 24 M keys) took 930 us in the two and that sum, now 742. Bound by their
+// counts and 64-bit offsets from a prefix sum over all rows: a 2048^3 mesh (30 M
+// rows, 39 M keys) took 930 us in the two and that sum, now 742. Bound by their
 // instructions: the row's box and centres and the tests of about three voxels.
 __global__ void __launch_bounds__(kThreads) row_count_kernel(const uint32_t *__restrict__ rowPair,
                                                              const PairBox *__restrict__ boxes,
@@ -1628,7 +1628,7 @@ __global__ void __launch_bounds__(kThreads) scan_down_kernel(const In *__restric
 // them a thread each, so that loads, stores and the work per head stay dense
 // (with eight neighbouring keys per thread, the threads' loads lay 64 bytes
 // apart and each thread went through its own heads: a 2048^3 mesh's segment
-// starts, 24 M keys, took 106 us where this takes 81, its two largest levels'
+// starts, 39 M keys, took 106 us where this takes 81, its two largest levels'
 // parents 128 + 45 and their sizes, in passes of their own, 15 + 19, where this
 // takes 55 + 37 for both). Bound by memory on the large levels, by its launches
 // on the small ones.
@@ -1839,8 +1839,8 @@ __global__ void widen_u32_kernel(const uint32_t *src, uint64_t *dst) { *dst = *s
 // reads up to 8 KB of sums that are in cache, where the pass in between is a
 // launch and one workgroup's work, on every scan and level of a small build: a
 // 256^3 mesh 950 us with it, 840 without, a 64^3 one 650 and 557, a 700^3 one
-// 2,565 and 2,490. Above, the sums read grow with the square of the blocks (24 M
-// keys: 11.5 K blocks, 0.5 GB) while the pass stays at 14 us.
+// 2,565 and 2,490. Above, the sums read grow with the square of the blocks (39 M
+// keys: 19 K blocks, 1.5 GB) while the pass stays at 14 us.
 constexpr uint64_t kDirectTiles = 1024;
 
 // The block sums of `bound` elements; `scan_sums` runs between the two passes.
@@ -2635,8 +2635,8 @@ static int mesh_core(Arena &ar, float *dv, int64_t nverts, int has_normals, int3
         if ((r = count_words(ar, total, 1))) return r;
         hipLaunchKernelGGL(row_count_kernel, dim3(unsigned(rowBlocks)), dim3(kThreads), 0, st, rowPair, boxes, ptri, rowStart,
                            R, pos, mp, marks, rowSums);
-        // one round of one workgroup, or the passes of their own: 72 K sums of
-        // a 2048^3 mesh took 84 us in 18 rounds, 10 in those
+        // one round of one workgroup, or the passes of their own: 119 K sums of
+        // a 2048^3 mesh took 84 us in 29 rounds, 10 in those
         if (rowBlocks <= uint64_t(kSumThreads) * kSumItems) {
             hipLaunchKernelGGL(scan_block_sums_kernel, dim3(1), dim3(kSumThreads), 0, st, rowSums, rowBlocks, total);
         } else {
