@@ -1136,12 +1136,6 @@ __global__ void root_init_kernel(LevelArrays root) {
     *root.cnt = 1;
 }
 
-__global__ void root_place_kernel(uint64_t *pos, uint64_t *B, uint32_t *bad) {
-    *pos = 0;
-    *B = 1;
-    *bad = 0;
-}
-
 // ---------------------------------------------------------------------------
 // signed-distance scene source (procedural replacement of the raw .voxel
 // route for SDF scenes; occupancy/normal rule of the workload definition)
@@ -1777,39 +1771,101 @@ __global__ void __launch_bounds__(kThreads) brick_emit_kernel(const uint32_t *__
 
 // A level's parents from the sorted child keys: parent j's key, first child,
 // child mask and subtree size (its children, at most 8 since keys are unique,
-// follow the head). Leaves have no sizes.
+// follow the head). Leaves have no sizes. One tile of child keys, its parents
+// from index j on; returns their count.
+template <bool Leaves>
+struct ParentTile {
+    uint64_t key[kScanTile + 8], size[Leaves ? 1 : kScanTile + 8];
+    uint16_t head[kScanTile];
+    uint32_t at[kScanItems * kThreads / 64];
+
+    __device__ __forceinline__ uint32_t emit(const LevelArrays &child, const LevelArrays &p, uint64_t n, uint64_t base,
+                                             uint64_t j) {
+        uint64_t bits[kScanItems];
+        tile_flags(child.key, base, n, 3, bits, key);
+        if (threadIdx.x < 8 && base + kScanTile + threadIdx.x < n)
+            key[kScanTile + threadIdx.x] = child.key[base + kScanTile + threadIdx.x];
+        if constexpr (!Leaves)
+            for (uint64_t q = threadIdx.x; q < kScanTile + 8; q += kThreads)
+                size[q] = child.S && base + q < n ? child.S[base + q] : 0;
+        const uint32_t heads = tile_heads(bits, head, at);
+        for (uint32_t h = threadIdx.x; h < heads; h += kThreads) {
+            const uint32_t i = head[h];
+            const uint64_t parent = key[i] >> 3;
+            uint32_t mask = 0, c = 0;
+            SubtreeSum sum;
+            for (; c < 8 && base + i + c < n; ++c) {
+                const uint64_t k = key[i + c];
+                if ((k >> 3) != parent) break;
+                mask |= 1u << uint32_t(k & 7);
+                if constexpr (!Leaves) sum.add(c, size[i + c]);
+            }
+            p.key[j + h] = parent;
+            p.start[j + h] = base + i;
+            p.mask[j + h] = mask | (sum.large(c) ? kLargeBit : 0);
+            p.S[j + h] = sum.size(c);
+        }
+        return heads;
+    }
+};
+
 template <bool Leaves>
 __global__ void __launch_bounds__(kThreads) parent_emit_kernel(LevelArrays child, LevelArrays p, TileSums t) {
-    __shared__ uint64_t key[kScanTile + 8], size[Leaves ? 1 : kScanTile + 8];
-    __shared__ uint16_t head[kScanTile];
-    __shared__ uint32_t at[kScanItems * kThreads / 64];
+    __shared__ ParentTile<Leaves> tile;
     __shared__ uint64_t lds[kThreads / 64];
     const uint64_t n = *child.cnt;
     const uint64_t base = uint64_t(blockIdx.x) * kScanTile;
     const uint64_t j = tile_offset(t, lds);
-    if (base >= n) return;
-    uint64_t bits[kScanItems];
-    tile_flags(child.key, base, n, 3, bits, key);
-    if (threadIdx.x < 8 && base + kScanTile + threadIdx.x < n)
-        key[kScanTile + threadIdx.x] = child.key[base + kScanTile + threadIdx.x];
-    if constexpr (!Leaves)
-        for (uint64_t q = threadIdx.x; q < kScanTile + 8; q += kThreads) size[q] = base + q < n ? child.S[base + q] : 0;
-    const uint32_t heads = tile_heads(bits, head, at);
-    for (uint32_t h = threadIdx.x; h < heads; h += kThreads) {
-        const uint32_t i = head[h];
-        const uint64_t parent = key[i] >> 3;
-        uint32_t mask = 0, c = 0;
-        SubtreeSum sum;
-        for (; c < 8 && base + i + c < n; ++c) {
-            const uint64_t k = key[i + c];
-            if ((k >> 3) != parent) break;
-            mask |= 1u << uint32_t(k & 7);
-            if constexpr (!Leaves) sum.add(c, size[i + c]);
+    if (base < n) tile.emit(child, p, n, base, j);
+}
+
+// The upper levels of a tree, up to kTopNodes nodes each, are one workgroup's
+// work in one launch, bottom-up and top-down: a launch of their own costs each
+// of them more than the work. Bound by the chain of its levels' reads; a 256^3
+// mesh 745 us with a launch or two per level, 709 so, a 64^3 one 465 and 418.
+constexpr uint64_t kTopNodes = 4096;
+constexpr int kMaxLevels = 22;
+struct Levels {
+    LevelArrays lv[kMaxLevels];
+    int n;
+};
+
+// lv[1], lv[2], ... from lv[0], each the parents of the one before. The barrier
+// between two levels orders their accesses: one workgroup, one compute unit.
+__global__ void __launch_bounds__(kThreads) top_parents_kernel(Levels l) {
+    __shared__ ParentTile<false> tile;
+    uint64_t n = *l.lv[0].cnt;
+    for (int k = 1; k < l.n; ++k) {
+        uint64_t parents = 0;
+        for (uint64_t base = 0; base < n; base += kScanTile) {
+            parents += tile.emit(l.lv[k - 1], l.lv[k], n, base, parents);
+            __syncthreads();
         }
-        p.key[j + h] = parent;
-        p.start[j + h] = base + i;
-        p.mask[j + h] = mask | (sum.large(c) ? kLargeBit : 0);
-        p.S[j + h] = sum.size(c);
+        if (threadIdx.x == 0) *l.lv[k].cnt = parents;
+        n = parents;
+    }
+}
+
+// The root's place, then the levels lv[0] (the root's), lv[1], ... but the last,
+// which gets its slots here and is written by a launch of its own, unless it is
+// the leaves' (leafWord: their words are written here).
+struct LevelCounts {
+    uint32_t n[kMaxLevels];
+};
+constexpr int kTopThreads = 1024;
+__global__ void __launch_bounds__(kTopThreads) write_top_kernel(Levels l, LevelCounts counts, const uint32_t *leafWord,
+                                                                uint32_t *out, uint64_t W, uint32_t *bad) {
+    if (threadIdx.x == 0) {
+        *l.lv[0].pos = 0;
+        *l.lv[0].B = 1;
+        *bad = 0;
+    }
+    __syncthreads();
+    for (int d = 0; d + 1 < l.n; ++d) {
+        const LevelArrays &child = l.lv[d + 1];
+        for (uint32_t k = threadIdx.x; k < counts.n[d]; k += kTopThreads)
+            write_node(k, l.lv[d], d + 2 == l.n ? leafWord : nullptr, child.S, child.pos, child.B, out, W, bad);
+        __syncthreads();
     }
 }
 
@@ -2123,6 +2179,21 @@ int emit_tree(Arena &ar, const Geometry &g, uint64_t *leafKey, uint32_t *leafWor
                 else hipLaunchKernelGGL(set_u64_kernel, dim3(1), dim3(1), 0, st, p.cnt, uint64_t(0));
                 continue;
             }
+            if (c.bound <= kTopNodes && !(multi && cacheLevel <= d)) {
+                Levels l;
+                l.n = 0;
+                l.lv[l.n++] = c;
+                for (int q = d; q >= 0; --q) {
+                    Level &t = lv[size_t(q)];
+                    t.bound = std::min(lv[size_t(q) + 1].bound, uint64_t(1) << (3 * q));
+                    if ((r = level_arrays(t, q == 0))) return r;
+                    l.lv[l.n++] = t;
+                }
+                hipLaunchKernelGGL(top_parents_kernel, dim3(1), dim3(kThreads), 0, st, l);
+                HIP_TRY(hipGetLastError());
+                for (int q = d + 1; q >= 0; --q) ar.release(lv[size_t(q)].key);
+                break;
+            }
             p.bound = d < 21 ? std::min(c.bound, uint64_t(1) << (3 * d)) : c.bound;
             if ((r = level_arrays(p, d == 0))) return r;
             // every parent below the count is written once (by its first child)
@@ -2180,8 +2251,18 @@ int emit_tree(Arena &ar, const Geometry &g, uint64_t *leafKey, uint32_t *leafWor
     for (int d = 0; d < D; ++d)
         if ((r = ar.alloc(lv[size_t(d)].pos, lv[size_t(d)].bound)) || (r = ar.alloc(lv[size_t(d)].B, lv[size_t(d)].bound)))
             return r;
-    hipLaunchKernelGGL(root_place_kernel, dim3(1), dim3(1), 0, st, lv[0].pos, lv[0].B, bad);
-    for (int d = 0; d < D; ++d) {
+    Levels top;
+    LevelCounts counts;
+    int first = 0;  // the first level with a launch of its own
+    for (; first < D && lv[size_t(first)].bound <= kTopNodes; ++first) {
+        top.lv[first] = lv[size_t(first)];
+        counts.n[first] = uint32_t(lv[size_t(first)].bound);
+    }
+    top.lv[first] = lv[size_t(first)];
+    top.n = first + 1;
+    hipLaunchKernelGGL(write_top_kernel, dim3(1), dim3(kTopThreads), 0, st, top, counts, first == D ? leafWord : nullptr, words,
+                       W, bad);
+    for (int d = first; d < D; ++d) {
         const Level &p = lv[size_t(d)], &c = lv[size_t(d) + 1];
         if (p.bound)
             hipLaunchKernelGGL(write_level_kernel, dim3(grid_for(p.bound)), dim3(kThreads), 0, st, LevelArrays(p), p.bound,

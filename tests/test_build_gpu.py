@@ -635,3 +635,19 @@ def test_rows_of_large_triangles(svo, golden, res, extent, threads):
     t = svo.VoxelOctree.build_from_mesh(tab, False, counts, idx, res, threads=threads, memory_budget=1 << 30)
     center, words, _ = orc.Mesh(tab, False, counts, idx).build(res, threads, 1 << 30)
     assert np.array_equal(t.words(), words) and np.array_equal(t.center(), center)
+
+
+@pytest.mark.parametrize("n", [2, 4095, 4096, 4097, 32768])
+def test_upper_levels_in_one_launch(svo, golden, n):
+    """Leaf counts around the size up to which levels share a launch, for trees
+    that lie in it whole and ones with levels below, against the oracle's build."""
+    rng = np.random.default_rng(100 + n)
+    for side, mem in ((32, 1 << 30), (64, 1 << 30), (64, 1 << 13)):
+        pick = rng.choice(side**3, n, replace=False)
+        vol = np.zeros(side**3, np.uint32)
+        vol[pick] = rng.integers(1, 2**32, n, dtype=np.uint32)
+        vol = vol.reshape(side, side, side)
+        print(f"[gpu] grid {side}^3 of {n} leaves mem={mem}", flush=True)
+        t = svo.VoxelOctree.build_from_grid(vol, memory_budget=mem)
+        center, words, _ = orc.build_grid(vol, mem)
+        assert np.array_equal(t.words(), words) and np.array_equal(t.center(), center)
