@@ -158,10 +158,10 @@ struct TriRow {
     bool out;
 
     static __device__ __forceinline__ bool apart(float pa, float pb, float rad) {
-        return (fminf(pa, pb) > rad) | (fmaxf(pa, pb) < -rad);
+        return int(fminf(pa, pb) > rad) | int(fmaxf(pa, pb) < -rad);
     }
     __device__ __forceinline__ bool wide(int k) const {
-        return (fminf(fminf(v0[k], v1[k]), v2[k]) > h[k]) | (fmaxf(fmaxf(v0[k], v1[k]), v2[k]) < -h[k]);
+        return int(fminf(fminf(v0[k], v1[k]), v2[k]) > h[k]) | int(fmaxf(fmaxf(v0[k], v1[k]), v2[k]) < -h[k]);
     }
     __device__ __forceinline__ TriRow(float cy, float cz, const float half[3], const float tv[9]) {
         const float c[3] = {0.0f, cy, cz};
@@ -177,7 +177,7 @@ struct TriRow {
             e1[k] = v2[k] - v1[k];
             e2[k] = v0[k] - v2[k];
         }
-        out = wide(1) | wide(2);
+        out = int(wide(1)) | int(wide(2));
         out |= apart(e0[2] * v0[1] - e0[1] * v0[2], e0[2] * v2[1] - e0[1] * v2[2], fabsf(e0[2]) * h[1] + fabsf(e0[1]) * h[2]);
         out |= apart(e1[2] * v0[1] - e1[1] * v0[2], e1[2] * v2[1] - e1[1] * v2[2], fabsf(e1[2]) * h[1] + fabsf(e1[1]) * h[2]);
         out |= apart(e2[2] * v0[1] - e2[1] * v0[2], e2[2] * v1[1] - e2[1] * v1[2], fabsf(e2[2]) * h[1] + fabsf(e2[1]) * h[2]);
@@ -209,7 +209,7 @@ struct TriRow {
             vmax[k] = nrm[k] > 0.0f ? b : a;
         }
         sep |= nrm[0] * vmin[0] + nrm[1] * vmin[1] + nrm[2] * vmin[2] > 0.0f;
-        return !sep & (nrm[0] * vmax[0] + nrm[1] * vmax[1] + nrm[2] * vmax[2] >= 0.0f);
+        return int(!sep) & int(nrm[0] * vmax[0] + nrm[1] * vmax[1] + nrm[2] * vmax[2] >= 0.0f);
     }
 };
 
