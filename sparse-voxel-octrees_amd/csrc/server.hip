@@ -894,7 +894,7 @@ int server_create(svo_octree *const *trees, int ntrees, const svo_server_config 
             return r;
         }
         maxDepth = std::max(maxDepth, t->depth);
-        s->wide = s->wide || t->words.size() >= (uint64_t(1) << 32);
+        s->wide = s->wide || wide_indices(t->words.size());
     }
     s->reg = reg_entries(maxDepth);
     s->stackSlots = lds_slots(maxDepth, s->reg);

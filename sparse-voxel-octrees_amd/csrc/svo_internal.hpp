@@ -153,6 +153,9 @@ struct PathLaunch {
     size_t lds;
 };
 PathLaunch path_launch(const svo_octree &h);
+// Whether kernels that step through ray_step, which holds word indices and
+// looks for far words everywhere, need 64-bit ones for a tree of that many words.
+inline bool wide_indices(uint64_t words) { return words >= (uint64_t(1) << 32); }
 int ensure_device(svo_octree &h);
 void release_device(svo_octree &h);
 int raymarch_device(svo_octree &h, int64_t n, const float *o, const float *d, const float *rs,

@@ -36,7 +36,7 @@ struct LaunchPlan {
     int slots = 1;
     int reg = 1;  // persistent form: stack entries held in registers
     int levels = 1;  // grid form: path entries of a wave's stack
-    bool wide = false, lod = false;
+    bool wide = false, lod = false;  // wide: the form's kernel takes 64-bit addresses (grid) or indices (persistent)
     size_t ldsPerBlock = 0;
     unsigned grid = 0;
     int refill = 16;
