@@ -93,6 +93,10 @@ struct Workspace {
     // Null if there was no memory to pin.
     static constexpr int kWords = 256;
     uint64_t *words = nullptr;
+    // One event per staging chunk, made by the first staged copy. They are the
+    // workspace's own because an event can only be recorded in streams of its device.
+    static constexpr int kEvents = 4;
+    hipEvent_t ev[kEvents] = {};
 };
 
 struct WorkspaceCache {
@@ -199,6 +203,8 @@ struct Arena {
             (void)hipStreamSynchronize(stream);
             (void)hipStreamDestroy(stream);
             if (ws->words) (void)hipHostFree(ws->words);
+            for (hipEvent_t e : ws->ev)
+                if (e) (void)hipEventDestroy(e);
             delete ws;
         } else {
             c.idle.push_back(ws);
@@ -2010,10 +2016,9 @@ struct Level : LevelArrays {  // the leaves' S, pos and B stay null
 // staging at a few GB/s).
 struct Staging {
     static constexpr uint64_t kChunk = uint64_t(8) << 20;  // bytes
-    static constexpr int kChunks = 4;
+    static constexpr int kChunks = Workspace::kEvents;
     std::mutex mu;
     void *buf[kChunks] = {};
-    hipEvent_t ev[kChunks] = {};
 };
 
 Staging &staging() {
@@ -2022,12 +2027,14 @@ Staging &staging() {
 }
 
 // toDevice: host -> pinned chunk -> device; else device -> pinned chunk -> host.
-int staged_copy(void *dev, void *host, uint64_t bytes, bool toDevice, hipStream_t st) {
+int staged_copy(Arena &ar, void *dev, void *host, uint64_t bytes, bool toDevice) {
     Staging &sg = staging();
     std::lock_guard<std::mutex> lock(sg.mu);
+    const hipStream_t st = ar.stream;
+    hipEvent_t *ev = ar.ws->ev;
     for (int k = 0; k < Staging::kChunks; ++k) {
         if (!sg.buf[k]) HIP_TRY(hipHostMalloc(&sg.buf[k], Staging::kChunk, hipHostMallocDefault));
-        if (!sg.ev[k]) HIP_TRY(hipEventCreateWithFlags(&sg.ev[k], hipEventDisableTiming));
+        if (!ev[k]) HIP_TRY(hipEventCreateWithFlags(&ev[k], hipEventDisableTiming));
     }
     uint8_t *d8 = static_cast<uint8_t *>(dev), *h8 = static_cast<uint8_t *>(host);
     const uint64_t n = (bytes + Staging::kChunk - 1) / Staging::kChunk;
@@ -2068,14 +2075,14 @@ int staged_copy(void *dev, void *host, uint64_t bytes, bool toDevice, hipStream_
         const int slot = int(j % Staging::kChunks);
         if (toDevice) e = hipMemcpyAsync(d8 + j * Staging::kChunk, sg.buf[slot], len_of(j), hipMemcpyHostToDevice, st);
         else e = hipMemcpyAsync(sg.buf[slot], d8 + j * Staging::kChunk, len_of(j), hipMemcpyDeviceToHost, st);
-        if (e == hipSuccess) e = hipEventRecord(sg.ev[slot], st);
+        if (e == hipSuccess) e = hipEventRecord(ev[slot], st);
     };
     if (!toDevice)
         for (uint64_t j = 0; j < std::min<uint64_t>(n, Staging::kChunks) && e == hipSuccess; ++j) dma(j);
     for (uint64_t j = 0; j < n && e == hipSuccess; ++j) {
         const int slot = int(j % Staging::kChunks);
         // download: chunk j has landed; upload: the chunk's previous DMA has left it
-        if (!toDevice || j >= uint64_t(Staging::kChunks)) e = hipEventSynchronize(sg.ev[slot]);
+        if (!toDevice || j >= uint64_t(Staging::kChunks)) e = hipEventSynchronize(ev[slot]);
         if (e != hipSuccess) break;
         ready.store(j + 1, std::memory_order_release);
         host_slice(j, 0);
@@ -2094,7 +2101,7 @@ int staged_copy(void *dev, void *host, uint64_t bytes, bool toDevice, hipStream_
 }
 
 // Copies W device words into out (sized to W by the caller or here).
-int download_words(const uint32_t *src, uint64_t W, WordVec &out, hipStream_t st) {
+int download_words(Arena &ar, const uint32_t *src, uint64_t W, WordVec &out) {
     if (out.size() != W) {
         try {
             out.resize(W);
@@ -2104,11 +2111,11 @@ int download_words(const uint32_t *src, uint64_t W, WordVec &out, hipStream_t st
     }
     const uint64_t bytes = W * sizeof(uint32_t);
     if (bytes <= Staging::kChunk) {
-        HIP_TRY(hipMemcpyAsync(out.data(), src, bytes, hipMemcpyDeviceToHost, st));
-        HIP_TRY(hipStreamSynchronize(st));
+        HIP_TRY(hipMemcpyAsync(out.data(), src, bytes, hipMemcpyDeviceToHost, ar.stream));
+        HIP_TRY(hipStreamSynchronize(ar.stream));
         return SVO_OK;
     }
-    return staged_copy(const_cast<uint32_t *>(src), out.data(), bytes, false, st);
+    return staged_copy(ar, const_cast<uint32_t *>(src), out.data(), bytes, false);
 }
 
 // Builds the word array from sorted, unique leaf keys/words. blockFlags marks
@@ -2283,7 +2290,7 @@ int emit_tree(Arena &ar, const Geometry &g, uint64_t *leafKey, uint32_t *leafWor
         return fail(SVO_ERR_DEVICE, std::string("builder: scatter: ") + hipGetErrorString(e));
     }
     if (!hostArray.get()) return fail(SVO_ERR_NOMEM, "builder: host word array");
-    if ((r = download_words(words, W, out.words, st))) return r;
+    if ((r = download_words(ar, words, W, out.words))) return r;
     int dev = 0;
     (void)hipGetDevice(&dev);
     guard.keep = true;
@@ -2552,7 +2559,7 @@ static int write_volume(Arena &ar, const Geometry &g, const MeshParams &mp, int 
                                nrm, col, mp, z0, sliceZ, word, count, bad);
         HIP_TRY(hipGetLastError());
         const uint64_t n = plane * uint64_t(std::min(sliceZ, g.dataD - z0));
-        if ((r = download_words(word, n, host, st))) return r;
+        if ((r = download_words(ar, word, n, host))) return r;
         if (std::fwrite(host.data(), 4, n, fp) != n) return fail(SVO_ERR_IO, "convert: short write");
     }
     uint32_t badH = 0;
@@ -2869,13 +2876,13 @@ struct UploadItem {
     const void *host;
     uint64_t bytes;
 };
-static int upload_arrays(const std::vector<UploadItem> &items, hipStream_t st, std::unique_lock<std::mutex> &lock) {
+static int upload_arrays(Arena &ar, const std::vector<UploadItem> &items, std::unique_lock<std::mutex> &lock) {
     uint64_t total = 0;
     for (const UploadItem &it : items) total += (it.bytes + kCarveAlign - 1) / kCarveAlign * kCarveAlign;
     if (total > Staging::kChunk) {
         for (const UploadItem &it : items)
             if (it.bytes)
-                if (int r = staged_copy(it.dev, const_cast<void *>(it.host), it.bytes, true, st)) return r;
+                if (int r = staged_copy(ar, it.dev, const_cast<void *>(it.host), it.bytes, true)) return r;
         return SVO_OK;
     }
     Staging &sg = staging();
@@ -2885,7 +2892,7 @@ static int upload_arrays(const std::vector<UploadItem> &items, hipStream_t st, s
     for (const UploadItem &it : items) {
         if (!it.bytes) continue;
         std::memcpy(p, it.host, it.bytes);
-        HIP_TRY(hipMemcpyAsync(it.dev, p, it.bytes, hipMemcpyHostToDevice, st));
+        HIP_TRY(hipMemcpyAsync(it.dev, p, it.bytes, hipMemcpyHostToDevice, ar.stream));
         p += (it.bytes + kCarveAlign - 1) / kCarveAlign * kCarveAlign;
     }
     return SVO_OK;
@@ -2954,10 +2961,11 @@ static int mesh_entry(const float *verts, int64_t nverts, int has_normals, const
             hipStream_t s;
             ~Drain() { (void)hipStreamSynchronize(s); }
         } drain{st};
-        if ((r = upload_arrays({{dv, verts, uint64_t(nverts) * 36},
+        if ((r = upload_arrays(ar,
+                               {{dv, verts, uint64_t(nverts) * 36},
                                 {dfc, face_counts, uint64_t(nfaces) * 4},
                                 {dfi, face_idx, uint64_t(at) * 4}},
-                               st, chunk)))
+                               chunk)))
             return r;
         uint32_t *flags, fh = 0;
         BoundPart *parts;
@@ -3105,7 +3113,7 @@ static int ply_entry(const char *path, int resolution, const svo_build_opts *opt
         return r;
     if ((r = fill32(flags, 1, 0, st))) return r;
     if (span > Staging::kChunk) {
-        if ((r = staged_copy(raw, const_cast<uint8_t *>(L.buf.data() + vbody), span, true, st))) return r;
+        if ((r = staged_copy(ar, raw, const_cast<uint8_t *>(L.buf.data() + vbody), span, true))) return r;
     } else {
         HIP_TRY(hipMemcpyAsync(raw, L.buf.data() + vbody, span, hipMemcpyHostToDevice, st));
     }

@@ -1,0 +1,46 @@
+// HIP entry points put in front of the runtime's for the builder's host-side
+// tests: loaded with RTLD_GLOBAL before libsvo_hip.so, whose calls then come
+// here first. All of them go on to the runtime.
+#include <dlfcn.h>
+#include <hip/hip_runtime_api.h>
+
+#include <algorithm>
+#include <map>
+#include <mutex>
+#include <set>
+
+namespace {
+
+std::mutex mu;
+std::map<hipEvent_t, std::set<hipStream_t>> recorded;
+std::set<hipStream_t> streams;
+
+template <typename F>
+F real(const char *name) {
+    void *h = dlopen("libamdhip64.so.7", RTLD_LAZY | RTLD_NOLOAD);
+    return reinterpret_cast<F>(dlsym(h, name));
+}
+
+}  // namespace
+
+extern "C" {
+
+// the most streams one event was recorded in; *distinct = streams recorded in
+int shim_streams_per_event(int *distinct) {
+    std::lock_guard<std::mutex> lock(mu);
+    size_t most = 0;
+    for (const auto &e : recorded) most = std::max(most, e.second.size());
+    *distinct = int(streams.size());
+    return int(most);
+}
+
+hipError_t hipEventRecord(hipEvent_t event, hipStream_t stream) {
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        recorded[event].insert(stream);
+        streams.insert(stream);
+    }
+    return real<decltype(&hipEventRecord)>("hipEventRecord")(event, stream);
+}
+
+}  // extern "C"
