@@ -5,6 +5,8 @@
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
+#include <chrono>
+#include <condition_variable>
 #include <map>
 #include <mutex>
 #include <set>
@@ -12,8 +14,13 @@
 namespace {
 
 std::mutex mu;
+std::condition_variable cv;
 std::map<hipEvent_t, std::set<hipStream_t>> recorded;
 std::set<hipStream_t> streams;
+
+int expected = 0, arrived = 0;
+bool late = false;
+thread_local bool met = false;
 
 template <typename F>
 F real(const char *name) {
@@ -41,6 +48,33 @@ hipError_t hipEventRecord(hipEvent_t event, hipStream_t stream) {
         streams.insert(stream);
     }
     return real<decltype(&hipEventRecord)>("hipEventRecord")(event, stream);
+}
+
+// From now on the first hipStreamSynchronize of each thread waits until
+// `threads` threads have come to theirs, 5 s at most.
+void shim_meet(int threads) {
+    std::lock_guard<std::mutex> lock(mu);
+    expected = threads;
+    arrived = 0;
+    late = false;
+}
+
+// whether they all came in time
+int shim_met() {
+    std::lock_guard<std::mutex> lock(mu);
+    return arrived == expected && !late;
+}
+
+hipError_t hipStreamSynchronize(hipStream_t stream) {
+    {
+        std::unique_lock<std::mutex> lock(mu);
+        if (expected && !met) {
+            met = true;
+            if (++arrived == expected) cv.notify_all();
+            else if (!cv.wait_for(lock, std::chrono::seconds(5), [] { return arrived == expected; })) late = true;
+        }
+    }
+    return real<decltype(&hipStreamSynchronize)>("hipStreamSynchronize")(stream);
 }
 
 }  // extern "C"

@@ -77,3 +77,32 @@ for _ in range(20):
         break
 assert distinct.value > 1 and most == 1, (distinct.value, most)
 """)
+
+
+def test_the_upload_chunk_goes_with_the_copies(shim):
+    """Two builds whose arrays fit the shared chunk together: each reaches its
+    first stream synchronisation while the other stands in its own, so neither
+    waits there with the chunk."""
+    print("[gpu] two builds at once, arrays of less than a staging chunk", flush=True)
+    _run(shim, """
+meshes = [mesh(20000, 1), mesh(20001, 2)]
+want = [expect(m) for m in meshes]
+assert all(m[0].nbytes + m[1].nbytes + m[2].nbytes < 1 << 23 and len(m[0]) + len(m[1]) >= 1 << 16 for m in meshes)
+at_once(meshes, 3)
+shim.shim_meet(2)
+got = at_once(meshes)
+assert shim.shim_met() == 1
+assert all(np.array_equal(g[0], words) for g, words in zip(got, want))
+""")
+
+
+def test_builds_at_once_on_every_upload_path(shim):
+    """Six threads, each its own mesh: host loops and pageable copies, the
+    device's checks with the shared chunk, and arrays of several chunks."""
+    print("[gpu] six builds at once", flush=True)
+    _run(shim, """
+meshes = [mesh(n, k) for k, n in enumerate((300, 9000, 16400, 30000, 60000, 70000))]
+want = [expect(m) for m in meshes]
+for got, words in zip(at_once(meshes, 5), want):
+    assert all(np.array_equal(g, words) for g in got)
+""")
