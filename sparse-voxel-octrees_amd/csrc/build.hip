@@ -2026,15 +2026,32 @@ Staging &staging() {
     return *s;
 }
 
+// A pinned chunk, or null: a build that finds no memory to pin copies from and
+// to pageable memory.
+void *pin_chunk() {
+    void *p = nullptr;
+    if (hipHostMalloc(&p, Staging::kChunk, hipHostMallocDefault) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+}
+
 // toDevice: host -> pinned chunk -> device; else device -> pinned chunk -> host.
 int staged_copy(Arena &ar, void *dev, void *host, uint64_t bytes, bool toDevice) {
     Staging &sg = staging();
-    std::lock_guard<std::mutex> lock(sg.mu);
+    std::unique_lock<std::mutex> lock(sg.mu);
     const hipStream_t st = ar.stream;
     hipEvent_t *ev = ar.ws->ev;
+    bool pinned = true;
     for (int k = 0; k < Staging::kChunks; ++k) {
-        if (!sg.buf[k]) HIP_TRY(hipHostMalloc(&sg.buf[k], Staging::kChunk, hipHostMallocDefault));
+        if (!sg.buf[k] && !(sg.buf[k] = pin_chunk())) pinned = false;
         if (!ev[k]) HIP_TRY(hipEventCreateWithFlags(&ev[k], hipEventDisableTiming));
+    }
+    if (!pinned) {
+        lock.unlock();
+        if (toDevice) HIP_TRY(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, st));
+        else HIP_TRY(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st));
+        HIP_TRY(hipStreamSynchronize(st));
+        return SVO_OK;
     }
     uint8_t *d8 = static_cast<uint8_t *>(dev), *h8 = static_cast<uint8_t *>(host);
     const uint64_t n = (bytes + Staging::kChunk - 1) / Staging::kChunk;
@@ -2871,7 +2888,7 @@ static int mesh_on_host(const float *verts, int64_t nverts, const int32_t *face_
 // Pinned chunks of Staging::kChunk bytes, one to a build at a time, at most
 // kKept of them kept for later builds. A build has its chunk until its stream
 // has passed the copies from it, kernels behind them included, so one chunk for
-// all made builds wait for each other: eight threads building meshes of 50 K
+// all made builds wait for each other: eight threads building meshes of 100 K
 // faces at 256^3, four each, took 8.8 ms so, now 8.0, four threads 5.4 and 5.0.
 // (One chunk with an event behind the copies, waited for by whoever takes it
 // next, cost every build 12-15 us.)
@@ -2897,17 +2914,17 @@ struct UploadChunk {
         if (p) (void)hipStreamSynchronize(stream);
         give();
     }
-    int take() {
+    bool take() {
         UploadChunks &c = upload_chunks();
         {
             std::lock_guard<std::mutex> lock(c.mu);
             if (c.n) {
                 p = c.idle[--c.n];
-                return SVO_OK;
+                return true;
             }
         }
-        HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&p), Staging::kChunk, hipHostMallocDefault));
-        return SVO_OK;
+        p = static_cast<char *>(pin_chunk());
+        return p != nullptr;
     }
     void give() {  // once no copy reads it
         if (!p) return;
@@ -2939,7 +2956,12 @@ static int upload_arrays(Arena &ar, const std::vector<UploadItem> &items, Upload
                 if (int r = staged_copy(ar, it.dev, const_cast<void *>(it.host), it.bytes, true)) return r;
         return SVO_OK;
     }
-    if (int r = chunk.take()) return r;
+    if (!chunk.take()) {
+        for (const UploadItem &it : items)
+            if (it.bytes) HIP_TRY(hipMemcpyAsync(it.dev, it.host, it.bytes, hipMemcpyHostToDevice, ar.stream));
+        HIP_TRY(hipStreamSynchronize(ar.stream));
+        return SVO_OK;
+    }
     char *p = chunk.p;
     for (const UploadItem &it : items) {
         if (!it.bytes) continue;

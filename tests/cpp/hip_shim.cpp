@@ -22,6 +22,8 @@ int expected = 0, arrived = 0;
 bool late = false;
 thread_local bool met = false;
 
+bool pinning = true;
+
 template <typename F>
 F real(const char *name) {
     void *h = dlopen("libamdhip64.so.7", RTLD_LAZY | RTLD_NOLOAD);
@@ -75,6 +77,14 @@ hipError_t hipStreamSynchronize(hipStream_t stream) {
         }
     }
     return real<decltype(&hipStreamSynchronize)>("hipStreamSynchronize")(stream);
+}
+
+// whether pinned memory can be had
+void shim_pinning(int on) { pinning = on; }
+
+hipError_t hipHostMalloc(void **ptr, size_t size, unsigned int flags) {
+    if (!pinning) return hipErrorOutOfMemory;
+    return real<hipError_t (*)(void **, size_t, unsigned int)>("hipHostMalloc")(ptr, size, flags);
 }
 
 }  // extern "C"

@@ -19,20 +19,20 @@ import numpy as np
 import conftest, oracle_py as orc
 svo = conftest.load_package()
 
-def mesh(faces, seed):
+def mesh(faces, seed, scale=0.01):
     rng = np.random.default_rng(seed)
     centre = rng.uniform(0.1, 0.9, (faces, 1, 3))
     tab = np.zeros((4 * faces, 9), np.float32)  # the fourth vertex is unused
-    tab[:, :3] = (centre + rng.normal(scale=0.01, size=(faces, 4, 3))).reshape(-1, 3)
+    tab[:, :3] = (centre + rng.normal(scale=scale, size=(faces, 4, 3))).reshape(-1, 3)
     tab[:, 6:] = 255.0
     idx = (4 * np.arange(faces)[:, None] + np.arange(3)).astype(np.int32).reshape(-1)
     return tab, np.full(faces, 3, np.int32), idx
 
-def build(m):
-    return svo.VoxelOctree.build_from_mesh(m[0], False, m[1], m[2], 64, threads=8, memory_budget=1 << 30).words()
+def build(m, res=64):
+    return svo.VoxelOctree.build_from_mesh(m[0], False, m[1], m[2], res, threads=8, memory_budget=1 << 30).words()
 
-def expect(m):
-    return orc.Mesh(m[0], False, m[1], m[2]).build(64, 8, 1 << 30)[1]
+def expect(m, res=64):
+    return orc.Mesh(m[0], False, m[1], m[2]).build(res, 8, 1 << 30)[1]
 
 def at_once(meshes, times=1):
     got = [[] for _ in meshes]
@@ -105,4 +105,19 @@ meshes = [mesh(n, k) for k, n in enumerate((300, 9000, 16400, 30000, 60000, 7000
 want = [expect(m) for m in meshes]
 for got, words in zip(at_once(meshes, 5), want):
     assert all(np.array_equal(g, words) for g in got)
+""")
+
+
+def test_builds_without_memory_to_pin(shim):
+    """Every copy path of a mesh build where no pinned memory is to be had: host
+    loops, the shared checks with one chunk's arrays, arrays of several chunks,
+    and a result of several."""
+    print("[gpu] builds without pinned memory", flush=True)
+    _run(shim, """
+cases = [(mesh(300, 1), 64), (mesh(20000, 2), 64), (mesh(60000, 3), 64), (mesh(9000, 4, 0.05), 256)]
+want = [expect(*c) for c in cases]
+assert want[-1].nbytes > 1 << 23
+shim.shim_pinning(0)
+for c, words in zip(cases, want):
+    assert np.array_equal(build(*c), words)
 """)
