@@ -41,6 +41,7 @@
 #include <vector>
 
 #include "build_common.hpp"
+#include "pinned_words.hpp"
 #include "range_alloc.hpp"
 #include "svo_internal.hpp"
 
@@ -87,12 +88,10 @@ struct Workspace {
     char *slab = nullptr;
     uint64_t size = 0;
     RangeAlloc fit;
-    // Pinned words in which the host receives counts: kernels write them there
-    // or one copy does. Into pageable memory each of a build's six round trips
-    // took a staging copy: a 256^3 mesh 855 us, now 741, a 64^3 one 550 and 454.
-    // Null if there was no memory to pin.
-    static constexpr int kWords = 256;
-    uint64_t *words = nullptr;
+    // The host receives counts in pinned words: kernels write them there or one
+    // copy does. Into pageable memory each of a build's six round trips took a
+    // staging copy: a 256^3 mesh 855 us, now 741, a 64^3 one 550 and 454.
+    PinnedWords words;
     // One event per staging chunk, made by the first staged copy. They are the
     // workspace's own because an event can only be recorded in streams of its device.
     static constexpr int kEvents = 4;
@@ -160,8 +159,8 @@ struct Arena {
                 return fail(SVO_ERR_DEVICE, std::string("builder: hipStreamCreate: ") + hipGetErrorString(e));
             }
             void *words = nullptr;
-            if (hipHostMalloc(&words, Workspace::kWords * sizeof(uint64_t), hipHostMallocCoherent) == hipSuccess)
-                ws->words = static_cast<uint64_t *>(words);
+            if (hipHostMalloc(&words, PinnedWords::kWords * sizeof(uint64_t), hipHostMallocCoherent) == hipSuccess)
+                ws->words.mem = static_cast<uint64_t *>(words);
             else
                 (void)hipGetLastError();
             hipMemPool_t pool;
@@ -169,6 +168,7 @@ struct Arena {
             if (default_pool(pool)) (void)hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep);
         }
         ws->fit.reset(ws->size);
+        ws->words.reset();
         stream = ws->stream;
         started = std::chrono::steady_clock::now();
         return SVO_OK;
@@ -202,7 +202,7 @@ struct Arena {
             if (ws->slab) (void)hipFreeAsync(ws->slab, stream);
             (void)hipStreamSynchronize(stream);
             (void)hipStreamDestroy(stream);
-            if (ws->words) (void)hipHostFree(ws->words);
+            if (ws->words.mem) (void)hipHostFree(ws->words.mem);
             for (hipEvent_t e : ws->ev)
                 if (e) (void)hipEventDestroy(e);
             delete ws;
@@ -1957,7 +1957,8 @@ int run_heads(Arena &ar, const uint64_t *keys, Count count, uint64_t bound, int 
 
 // Reads device words into host values in one copy (one round trip).
 int read_words(Arena &ar, const uint64_t *src, uint64_t *dst, int count, hipStream_t s) {
-    uint64_t *land = ar.ws->words && count <= Workspace::kWords ? ar.ws->words : dst;
+    uint64_t *land = ar.ws->words.land(count);
+    if (!land) land = dst;
     HIP_TRY(hipMemcpyAsync(land, src, sizeof(uint64_t) * count, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
     if (land != dst) std::memcpy(dst, land, sizeof(uint64_t) * count);
@@ -1965,23 +1966,20 @@ int read_words(Arena &ar, const uint64_t *src, uint64_t *dst, int count, hipStre
 }
 
 // `count` words that kernels write and the host reads next (read_counts): the
-// workspace's pinned words, one set at a time, or device memory.
+// workspace's pinned words if they are free, or device memory.
 int count_words(Arena &ar, uint64_t *&w, int count) {
-    if (ar.ws->words && count <= Workspace::kWords) {
-        w = ar.ws->words;
-        return SVO_OK;
-    }
-    return ar.alloc(w, uint64_t(count));
+    w = ar.ws->words.take(count);
+    return w ? SVO_OK : ar.alloc(w, uint64_t(count));
 }
 int read_counts(Arena &ar, uint64_t *w, uint64_t *dst, int count, hipStream_t s) {
-    if (w != ar.ws->words) {
+    if (w != ar.ws->words.mem) {
         if (int r = read_words(ar, w, dst, count, s)) return r;
         ar.release(w);
         return SVO_OK;
     }
     HIP_TRY(hipStreamSynchronize(s));
     std::memcpy(dst, w, sizeof(uint64_t) * count);
-    return SVO_OK;
+    return ar.ws->words.give(w) ? SVO_OK : fail(SVO_ERR_DEVICE, "builder: count words given back twice (internal error)");
 }
 
 // Exclusive scan whose total the host needs next.
@@ -2293,7 +2291,8 @@ int emit_tree(Arena &ar, const Geometry &g, uint64_t *leafKey, uint32_t *leafWor
                                LevelArrays(c), d == D - 1 ? leafWord : nullptr, words, W, bad);
     }
     uint32_t badH = 0;
-    uint32_t *badLand = ar.ws->words ? reinterpret_cast<uint32_t *>(ar.ws->words) : &badH;
+    uint64_t *badWord = ar.ws->words.land(1);
+    uint32_t *badLand = badWord ? reinterpret_cast<uint32_t *>(badWord) : &badH;
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpyAsync(badLand, bad, 4, hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
