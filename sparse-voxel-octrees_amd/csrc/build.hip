@@ -2241,11 +2241,12 @@ int emit_tree(Arena &ar, const Geometry &g, uint64_t *leafKey, uint32_t *leafWor
     const uint64_t W = 1 + report[size_t(D) + 1];
     // the word array, allocated before the host array below: both map memory
     // into the process, and a device allocation waits while other threads
-    // populate host pages
+    // populate host pages; with the spare word of every device array
+    // (kSpareWords)
     uint32_t *words;
     {
         void *pw = nullptr;
-        hipError_t e = hipMalloc(&pw, W * sizeof(uint32_t));
+        hipError_t e = hipMalloc(&pw, (W + kSpareWords) * sizeof(uint32_t));
         if (e != hipSuccess) return fail(SVO_ERR_NOMEM, std::string("builder: word array: ") + hipGetErrorString(e));
         words = static_cast<uint32_t *>(pw);
     }

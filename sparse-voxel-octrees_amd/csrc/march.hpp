@@ -512,7 +512,7 @@ SVO_HD int walk(const Ray<Addr> &r, const uint32_t *__restrict__ tree, const Pat
             SVO_HOLD("+v"(width));
             const Addr p = ((Addr(sib) << width) + block) & ~Addr(3);
             // a two-word slot's far word travels with its descriptor (device
-            // arrays have a word to spare after the last)
+            // arrays have a word to spare after the last, kSpareWords)
             const bool two = width == 3;
             uint32_t farWord;
             m = tree_word<Addr>(tree, p);

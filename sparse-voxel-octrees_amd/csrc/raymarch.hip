@@ -261,9 +261,7 @@ int ensure_device(svo_octree &h) {
     release_device(h);
     size_t bytes = h.words.size() * sizeof(uint32_t);
     void *p = nullptr;
-    // one word more than the tree: the walk reads the word after a two-word
-    // slot's descriptor, which a tree from a file may end with
-    hipError_t e = hipMalloc(&p, bytes + sizeof(uint32_t));
+    hipError_t e = hipMalloc(&p, bytes + kSpareWords * sizeof(uint32_t));
     if (e != hipSuccess) return fail(SVO_ERR_NOMEM, std::string("hipMalloc octree: ") + hipGetErrorString(e));
     e = hipMemcpy(p, h.words.data(), bytes, hipMemcpyHostToDevice);
     if (e != hipSuccess) {

@@ -156,6 +156,9 @@ PathLaunch path_launch(const svo_octree &h);
 // Whether kernels that step through ray_step, which holds word indices and
 // looks for far words everywhere, need 64-bit ones for a tree of that many words.
 inline bool wide_indices(uint64_t words) { return words >= (uint64_t(1) << 32); }
+// Device word arrays are that much longer than their trees: the walk reads the
+// word after a two-word slot's descriptor, with which a tree from a file may end.
+constexpr uint64_t kSpareWords = 1;
 int ensure_device(svo_octree &h);
 void release_device(svo_octree &h);
 int raymarch_device(svo_octree &h, int64_t n, const float *o, const float *d, const float *rs,

@@ -102,3 +102,18 @@ def test_every_tile_runs_once_around_the_run_length(svo, golden, tiles):
     ren = svo.svo.Renderer(2)
     ren.render_device([ren.view(tree, cam, w, h, **ptr)])
     _same(got(), ref, "batch")
+
+
+def test_device_arrays_have_a_word_to_spare(svo, golden):
+    """The walk reads the word after a two-word slot's descriptor: the device
+    arrays of built trees and of trees from words are longer than the trees."""
+    import ctypes
+    import torch
+    assert torch.cuda.is_available()
+    hip = ctypes.CDLL("libamdhip64.so.7")  # the runtime in use, by its soname
+    vol = np.random.default_rng(2).integers(1, 2**32, (40, 40, 40), dtype=np.uint32)
+    built = svo.VoxelOctree.build_from_grid(vol)
+    for what, tree in (("built", built), ("from words", svo.VoxelOctree.from_words(built.words(), built.center()))):
+        base, size = ctypes.c_void_p(), ctypes.c_size_t()
+        assert hip.hipMemGetAddressRange(ctypes.byref(base), ctypes.byref(size), ctypes.c_void_p(tree.upload())) == 0
+        assert size.value >= 4 * (tree.word_count() + 1), what
