@@ -34,3 +34,17 @@ def test_walk_equals_the_reference_loop(walk_test, golden, tmp_path, tree):
     r = subprocess.run([walk_test, path, str(levels), "20000"] + (["loose"] if tree.startswith("loose") else []), capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stdout + r.stderr
     assert r.stdout.startswith("ok ")
+
+
+@pytest.mark.parametrize("levels,seed,loose", [(1, 2, False), (2, 2, False), (3, 3, False), (10, 10, False), (23, 23, False),
+                                               (3, 3, True), (10, 10, True)])
+def test_compared_walks_end_in_leaves_and_cut_offs(walk_test, tmp_path, levels, seed, loose):
+    """The comparison above is of rays of every outcome: at least a tenth of its
+    walks end in a leaf and a hundredth at a cut-off, misses are the rest."""
+    path = str(tmp_path / "words.bin")
+    mixed_tree(seed, levels, loose=loose).tofile(path)
+    r = subprocess.run([walk_test, path, str(levels), "20000"] + (["loose"] if loose else []), capture_output=True, text=True,
+                       timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
+    walks, leaves, cuts = (int(r.stdout.split()[k]) for k in (1, 3, 6))
+    assert leaves >= walks / 10 and cuts >= walks / 100 and walks - leaves - cuts >= walks / 100, r.stdout

@@ -117,3 +117,87 @@ def test_device_arrays_have_a_word_to_spare(svo, golden):
         base, size = ctypes.c_void_p(), ctypes.c_size_t()
         assert hip.hipMemGetAddressRange(ctypes.byref(base), ctypes.byref(size), ctypes.c_void_p(tree.upload())) == 0
         assert size.value >= 4 * (tree.word_count() + 1), what
+
+
+def _device_outputs(n):
+    import torch
+    return {k: torch.full((n,), 7, dtype=dt, device="cuda")
+            for k, dt in (("hit", torch.uint8), ("normal", torch.int32), ("t", torch.float32), ("leaf", torch.int64))}
+
+
+def _fetch(out):
+    """The outputs on the host; filled again for the next launch."""
+    import torch
+    torch.cuda.synchronize()
+    r = {"hit": out["hit"].cpu().numpy(), "normal": out["normal"].cpu().numpy().view(np.uint32), "t": out["t"].cpu().numpy(),
+         "leaf": out["leaf"].cpu().numpy().view(np.uint64)}
+    for v in out.values():
+        v.fill_(7)
+    torch.cuda.synchronize()
+    return r
+
+
+@pytest.mark.parametrize("levels", [3, 10])
+def test_wide_walk_through_plans_shadows_and_mixed_batches(svo, levels):
+    """The 64-bit walk (a loose tree's) in the planned primary, shadow, frame and
+    batch launches; in a batch it carries a tight tree's views along. Plans run
+    three times: raster order, then filed orders."""
+    import torch
+    loose, tight = mixed_tree(levels, levels, loose=True), mixed_tree(levels, levels)
+    centre = np.full(3, 0.5, np.float32)
+    trees = {"loose": svo.VoxelOctree.from_words(loose, centre), "tight": svo.VoxelOctree.from_words(tight, centre)}
+    words = {"loose": loose, "tight": tight}
+    w, h, eps = 203, 131, 0.01
+    light = np.array([0.3, 0.8, 0.2], np.float32)
+    tree = trees["loose"]
+    cam = tree.orbit_camera(25.0, 40.0, 1.0)
+    tf, pos = np.frombuffer(cam.tform, np.float32), np.frombuffer(cam.pos, np.float32)
+    dirs = orc.primary_dirs(tf, w, h)
+    prim = {k: orc.raymarch(v, pos[None, :], dirs, 0.0) for k, v in words.items()}
+    cut = {k: orc.raymarch(v, pos[None, :], dirs, 0.02) for k, v in words.items()}
+    hit = prim["loose"]["hit"] == 1
+    assert hit.mean() > 0.3 and (levels == 3 or (cut["loose"]["hit"] == 2).any())
+    o = (pos[None, :] + dirs[hit] * (prim["loose"]["t"][hit] - np.float32(eps))[:, None]).astype(np.float32)
+    shadow = np.zeros(w * h, np.uint8)
+    shadow[hit] = orc.raymarch(loose, o, np.broadcast_to(light, o.shape).copy(), 0.0)["hit"] != 0
+    assert 0.1 < shadow[hit].mean() < 0.9
+    print(f"[gpu] wide walk: {levels} levels, planned primary", flush=True)
+    out = _device_outputs(w * h)
+    p = {k: v.data_ptr() for k, v in out.items()}
+    plan = svo.svo.TilePlan(w, h)
+    for k in range(3):
+        plan.render_device(tree, cam, p["hit"], p["normal"], p["t"], p["leaf"])
+        _same(_fetch(out), prim["loose"], ("planned", k))
+    print("[gpu] wide walk: shadows", flush=True)
+    sh = torch.full((w * h,), 7, dtype=torch.uint8, device="cuda")
+    splan = svo.svo.TilePlan(w, h)
+    for k, pl in enumerate((None, splan, splan, splan)):
+        tree.render_shadow_device(cam, w, h, light, eps, p["hit"], p["t"], sh.data_ptr(), p["normal"], p["leaf"], plan=pl)
+        _same(_fetch(out), prim["loose"], ("shadow primary", k))
+        assert np.array_equal(sh.cpu().numpy(), shadow), ("shadow", k)
+        sh.fill_(7)
+    print("[gpu] wide walk: frames", flush=True)
+    fw, fh = 208, 128
+    ref_rgba, ref_depth = orc.render_frame(loose, tf, centre, fw, fh, 16, 1)
+    rgba = torch.zeros(fw * fh, dtype=torch.int32, device="cuda")
+    depth = torch.zeros(svo.svo.frame_depth_count(fw, fh, 16), dtype=torch.float32, device="cuda")
+    fplan = svo.svo.TilePlan.for_frame(fw, fh, 16)
+    for k, pl in enumerate((None, fplan, fplan, fplan)):
+        tree.render_frame_device(cam, fw, fh, rgba.data_ptr(), depth.data_ptr(), 16, 1, plan=pl)
+        torch.cuda.synchronize()
+        assert np.array_equal(rgba.cpu().numpy().view(np.uint32).reshape(-1), np.asarray(ref_rgba).reshape(-1)), k
+        assert np.array_equal(depth.cpu().numpy().view(np.uint32), np.asarray(ref_depth).reshape(-1).view(np.uint32)), k
+        rgba.zero_()
+        depth.zero_()
+    print("[gpu] wide walk: batches", flush=True)
+    ren = svo.svo.Renderer(4)
+    for scales in ((0.0, 0.0), (0.0, 0.02), (0.02, 0.0)):
+        outs = [_device_outputs(w * h) for _ in range(2)]
+        views = [ren.view(trees[n], cam, w, h, ray_scale=rs, **{k: v.data_ptr() for k, v in out.items()})
+                 for n, rs, out in zip(("loose", "tight"), scales, outs)]
+        refs = [(cut if rs else prim)[n] for n, rs in zip(("loose", "tight"), scales)]
+        bplan = svo.svo.TilePlan.for_batch(views)
+        for k, opts in enumerate(({}, {"form": svo.svo.BATCH_PERSISTENT}, {"plan": bplan}, {"plan": bplan}, {"plan": bplan})):
+            ren.render_device(views, **opts)
+            for out, ref in zip(outs, refs):
+                _same(_fetch(out), ref, ("batch", scales, k))
