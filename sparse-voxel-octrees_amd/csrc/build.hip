@@ -23,9 +23,10 @@
 //   - above the cache-block level occupancy comes from the top table, so a
 //     cache block counted non-empty but holding no voxel still becomes an
 //     (empty) node.
-//  then levels bottom-up (parent = key >> 3, child masks), subtree sizes with
-//  the far-pointer rule, offsets top-down, and a scatter of every word into
-//  the depth-first layout (see size_kernel / place_kernel).
+//  then levels bottom-up (parent = key >> 3, child masks, subtree sizes with
+//  the far-pointer rule: SubtreeSum, ParentTile), and top-down, in one pass per
+//  level, the children's places and the level's words in the depth-first
+//  layout (write_node).
 #include <hip/hip_runtime.h>
 #include <rocprim/device/device_radix_sort.hpp>
 

@@ -150,8 +150,10 @@ __device__ __forceinline__ bool tri_box(const float c[3], const float h[3], cons
 // three tests about the x axis and the box's y and z extents, which also rule
 // out whole rows; the six other axis tests, the x extent and the plane remain
 // per voxel, without a branch between them. A mesh's vertices lie in the unit
-// cube by then, so nothing here is a NaN and minimum and maximum stand for the
-// comparisons they are made of.
+// cube by then, so that no product overflows and minimum and maximum stand for
+// the comparisons they are made of. NaNs come only from an extent beyond the
+// largest float, and a triangle with one overlaps nothing in either form: two
+// components of its normal are NaN, and the last test fails.
 struct TriRow {
     float v0[3], v1[3], v2[3], e0[3], e1[3], e2[3], tx[3];  // [0] per voxel, x from tx
     float h[3], n0;

@@ -5,11 +5,14 @@
 // results are bit-identical to the reference on the same rays. Design:
 //  - one lane per ray; a wave64 owns an 8x8 pixel tile (render path) so its
 //    rays walk the same nodes and its node loads coalesce through L2;
-//  - the restart stack {parent, maxT} per scale lives in LDS, laid out
-//    [slot][lane] so a wave's pushes/pops hit 64 different banks;
+//  - the nodes on a ray's path (child block and masks per level, PathStack)
+//    live in LDS, laid out [level][lane] so a wave's accesses hit different
+//    banks; rays that are not finite take the reference's loop, whose
+//    {parent, maxT} stack lies in the same LDS but for its top entries;
 //  - node words are fetched with plain 32-bit global loads (the tree is
 //    read-only, so they stay cached in L2 / MALL across rays);
-//  - word indices are 32-bit when the tree has < 2^32 words, else 64-bit.
+//  - words are addressed by 32-bit byte offsets when the tree has < 2^30
+//    words and far words in two-word slots only, else by 64-bit ones (path_launch).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -62,6 +65,9 @@ __device__ __forceinline__ void store_result(int code, uint32_t normal, float t,
 
 // Arbitrary caller rays, one wave per 64: finite rays take the walk, the
 // others the reference's loop step by step (exact std::min and NaN semantics).
+// A wave with both kinds lays both their stacks over the same LDS: one side of
+// the branch ends, its outcome in registers, before the other begins, and
+// neither reads an entry that its own lane has not put there.
 template <bool Lod, typename Addr>
 __global__ void __launch_bounds__(64) rays_kernel(const uint32_t *__restrict__ tree, int64_t n,
                                                   const float *__restrict__ o, const float *__restrict__ d,

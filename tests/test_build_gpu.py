@@ -651,3 +651,22 @@ def test_upper_levels_in_one_launch(svo, golden, n):
         t = svo.VoxelOctree.build_from_grid(vol, memory_budget=mem)
         center, words, _ = orc.build_grid(vol, mem)
         assert np.array_equal(t.words(), words) and np.array_equal(t.center(), center)
+
+
+@pytest.mark.parametrize("n", [300, 20000])
+@pytest.mark.parametrize("flat", [False, True])
+def test_mesh_extents_beyond_the_largest_float(svo, golden, n, flat):
+    """Extents that overflow scale every vertex to zero or NaN; triangles with a
+    NaN overlap no voxel. By host checks and by the device's, against the oracle."""
+    rng = np.random.default_rng(4)
+    tab = np.zeros((4 * n, 9), np.float32)
+    tab[:, 6:] = 200.0
+    tab[:, :3] = rng.uniform(-3.4e38, 3.4e38, (4 * n, 3))
+    tab[: 2 * n, :3] = rng.uniform(-3.4e38, -3.0e38, (2 * n, 3))
+    if flat:
+        tab[:, 1:3] = rng.uniform(0, 1, (4 * n, 2))
+    counts, idx = np.full(n, 3, np.int32), rng.integers(0, 4 * n, 3 * n).astype(np.int32)
+    print(f"[gpu] mesh of {n} faces, extent beyond float", flush=True)
+    t = svo.VoxelOctree.build_from_mesh(tab, False, counts, idx, 64, threads=8, memory_budget=1 << 30)
+    center, words, _ = orc.Mesh(tab, False, counts, idx).build(64, 8, 1 << 30)
+    assert np.array_equal(t.words(), words) and np.array_equal(t.center(), center)
